@@ -110,25 +110,30 @@ struct SorLevels {
   std::vector<int32_t> ptr;
 };
 
-// plan of a triangular sweep (SOR sweeps, IC / ILU solves): rows in level
-// order, rec[k] = {row, first, end, 0} of its dependency entries, packed in
-// the row's order: dcol = the column read, dent = the entry (position in the
-// values / factor) whose coefficient multiplies it
+// plan of a triangular sweep (SOR sweeps, IC / ILU solves; layout and reasons
+// in trisolve.hip): the rows in sweep order (rev: last row first) are cut
+// into chunks of crows consecutive rows and each chunk into one range per
+// wave; d_row lists the rows wave by wave, each wave's by level, d_hdr a
+// wave's batches, d_slot / d_dent their entries
 struct TriPlan {
   bool built = false;
-  SorLevels lev;  // d_rows = the rows in level order
-  int4 *d_rec = nullptr;
-  // dpos: level-order position of the row read, or -1 when the sweep's LDS
-  // copy of it may already be overwritten
-  int32_t *d_dcol = nullptr, *d_dent = nullptr, *d_dpos = nullptr;
-  int64_t ndeps = 0;
-  // blocks of whole levels staged through LDS: {first level, first
-  // position, first dependency entry}, nblk + 1 entries (0: not staged)
-  int4 *d_blk = nullptr;
-  int32_t nblk = 0;
-  // dependency-driven sweep across the chip (ticket: its work counter)
-  bool flow = false;
+  SorLevels lev;  // d_rows = the rows in level order (the factorisation's schedule)
+  int64_t n = 0, ndeps = 0, nrow = 0;  // ndeps, nrow: with padding
+  int32_t crows = 0, nchunk = 0, rev = 0, width = 0;  // width: entries per row and batch
+  int4 *d_hdr = nullptr;
+  uint16_t *d_slot = nullptr;  // LDS slot of the value that an entry reads
+  int32_t *d_dent = nullptr;   // position of its coefficient in the values / factor, or -1
+  int32_t *d_row = nullptr;
+  int32_t *d_ext = nullptr;    // rows of earlier chunks, in the order the waves take them
+  // per wave: first batch, first row of d_slot / d_dent, first of d_row, first of d_ext; one
+  // more at the end
+  int64_t *d_wave = nullptr;
   uint32_t *d_ticket = nullptr;
+  // dependency-driven form (scattered matrices): the rows in level order,
+  // {row, first entry, end}, d_dent in the same order, the columns read
+  bool flow = false;
+  int4 *d_rec = nullptr;
+  int32_t *d_dcol = nullptr;
 };
 // plans of a matrix: entries left of the diagonal; left of it up to the
 // first other entry (the SOR solver's sweep); right of it; rows of L^T (IC,
@@ -137,11 +142,11 @@ enum { kTriLower = 0, kTriLowerBreak = 1, kTriUpper = 2, kTriLt = 3 };
 // how a row ends: out = acc * sc; the SOR backward form (acc in double
 // from 0, out -= acc * sc); out = acc / sc; out = acc
 enum { kTriMul = 0, kTriSorBack = 1, kTriDiv = 2, kTriUnit = 3 };
-// a plan with its coefficients and per-row scale gathered in level order
+// a plan with its coefficients, and the initial value and scale of each row,
+// gathered in its order
 struct TriOp {
   const TriPlan *plan = nullptr;
-  void *coef = nullptr, *sc = nullptr;
-  void *ginit = nullptr;  // staged and flow plans: the initial values in level order
+  void *coef = nullptr, *isc = nullptr;
   int fin = kTriMul;
 };
 
@@ -390,16 +395,16 @@ void build_tri_plan(const std::vector<int32_t> &ptr, const std::vector<int32_t> 
 // plan kTriLower / kTriLowerBreak / kTriUpper of A's pattern, built on first
 // use from the device row_ptr / col_ind
 const TriPlan &tri_plan(Csr *A, int which);
-// gather coef[d] = vals[dent[d]] and sc[k] = scale[scale_pos ? scale_pos[row]
-// : row] for the plan (buffers from the context's scratch)
+// gather the coefficients vals[dent[d]] and the scales scale[scale_pos ?
+// scale_pos[row] : row] for the plan (buffers from the context's scratch)
 TriOp tri_prepare(Csr *A, const TriPlan &P, mgx_dtype dt, int fin, const void *vals,
                   const void *scale, const int32_t *scale_pos);
 // one sweep: out_row = fin(in_row - sum coef * out_col) in level order
 void tri_run(Csr *A, const TriOp &op, mgx_dtype dt, const void *in, void *out);
 void levels_free(SorLevels &L);
 void tri_free(Csr *A);
-// throws MGX_ERR_TIMEOUT (and clears the flag) when a dependency-driven sweep
-// of one of A's plans gave up since the last check
+// throws MGX_ERR_TIMEOUT (and clears the flag) when a sweep of one of A's plans
+// gave up since the last check
 void tri_check_stall(Csr *A);
 // IC(0) (kind MGX_PRECOND_IC) / ILU(0) (MGX_PRECOND_ILU) of A's pattern:
 // f (A->nnz entries of dt) holds a copy of the values on entry and the

@@ -1,20 +1,42 @@
-// trisolve.hip -- level-scheduled triangular sweeps: the SOR sweeps
+// trisolve.hip -- triangular sweeps: the SOR sweeps
 // (src/equation/kernel/sor_kernel.hpp:5-73) and the IC / ILU triangular
 // solves (csrsv2 in kernel/ic_kernel.hpp, ilu_kernel.hpp).
 //
 // Every such sweep has one form: out_i = fin(init_i - sum_d coef_d *
 // out_{col_d}), the sum over the row's dependency entries in the row's
-// storage order.  A plan, built once per matrix structure, lists the rows
-// in level order (level of a row = 1 + the largest level of the rows it
-// reads) with their dependency entries packed behind each other, so a row
-// needs one 16-byte record and contiguous entry loads; the coefficients and
-// the per-row scale are gathered into the same order once per solve.  Rows
-// of a level are independent and each row does the serial loop's
-// arithmetic in its order, so the result is bit-identical to the serial
-// sweep.  Within a row the entries are loaded eight at a time before their
-// products are subtracted in order, so a row costs a few memory round
-// trips, not two per entry.
+// storage order.  Each row does the serial loop's arithmetic in its order,
+// so the result is bit-identical to the serial sweep.
+//
+// A sweep is one serial chain of rows as long as the matrix has levels
+// (level of a row = 1 + the largest level of the rows it reads), so what
+// bounds it is the time from one row's value to the row that reads it, not
+// bandwidth: 2D Poisson 256^2 has 511 levels, 27-point 96^3 has 666.  The
+// plan therefore keeps that step inside one wave or one workgroup wherever
+// it can.  Rows are cut into chunks of consecutive rows in sweep order, one
+// workgroup each, and a chunk into the ranges of its kChWaves waves:
+//  - a wave runs its rows by level, the rows of a level side by side, with
+//    no barrier: its own values come back through LDS in program order;
+//  - a value of another wave of the chunk is read from LDS too, where a
+//    marker (a signalling NaN) says that it is not there yet;
+//  - a value of an earlier chunk is loaded from global memory ahead of its
+//    first use and kept in a ring of the wave in LDS.
+// Chunks are taken in sweep order and read only earlier ones, so they are
+// done or running: the sweep cannot deadlock, however few workgroups run.
+//
+// A wave runs alone on its SIMD, so a level costs its instructions (about
+// five clocks each) and one LDS round trip of 64 clocks, and the four waves
+// share one vector memory unit (16 clocks a load).  The plan is therefore
+// laid out in batches of up to 64 rows of several levels, one row per lane:
+// a batch is loaded once, a few batches ahead, and each of its levels only
+// reads its values from LDS, adds and writes.  Rows are filled up to D
+// entries with coefficient 0 and a slot that holds 0 (x - 0 * 0 is x, bit
+// for bit, but for a signalling NaN, which turns quiet: no row ever equals
+// the marker); a row of more than D entries takes several batches.  A
+// missing value shows as a NaN in the sum, so levels that miss nothing
+// compare nothing else.
 #include <algorithm>
+#include <functional>
+#include <future>
 #include <vector>
 
 #include "mgx_device.hpp"
@@ -24,407 +46,363 @@ namespace mgx {
 
 namespace {
 
-constexpr int kTriChunk = 8;
-// level-order positions whose values the single-workgroup sweeps keep in
-// LDS (a read of an older position goes to out)
-constexpr int kTriRing = 4096;
-
-// FIN 0: out = acc * sc (SOR forward); 1: SOR backward, acc in double from
-// 0, out = (T)((double)out - acc * (double)sc); 2: out = acc / sc; 3: out = acc
-template <class T, int FIN>
-__device__ __forceinline__ void tri_row(const int4 rc, const int32_t *__restrict__ dcol,
-                                        const T *__restrict__ dcoef, const T scv,
-                                        const T *__restrict__ in, T *out) {
-  const int32_t i = rc.x, d0 = rc.y, d1 = rc.z;
-  using Acc = typename std::conditional<FIN == 1, double, T>::type;
-  Acc acc = (Acc)0;
-  if (FIN != 1) acc = (Acc)in[i];
-  for (int32_t d = d0; d < d1; d += kTriChunk) {
-    int32_t c[kTriChunk];
-    T a[kTriChunk], zv[kTriChunk];
-#pragma unroll
-    for (int u = 0; u < kTriChunk; u++) {
-      c[u] = d + u < d1 ? dcol[d + u] : i;
-      a[u] = d + u < d1 ? dcoef[d + u] : (T)0;
-    }
-#pragma unroll
-    for (int u = 0; u < kTriChunk; u++) zv[u] = d + u < d1 ? out[c[u]] : (T)0;
-#pragma unroll
-    for (int u = 0; u < kTriChunk; u++) {
-      if (d + u < d1) {
-        const T p = a[u] * zv[u];
-        if (FIN == 1)
-          acc = acc + (double)p;
-        else
-          acc = acc - p;
-      }
-    }
-  }
-  if (FIN == 0)
-    out[i] = acc * scv;
-  else if (FIN == 1)
-    out[i] = (T)((double)out[i] - acc * (double)scv);
-  else if (FIN == 2)
-    out[i] = acc / scv;
-  else
-    out[i] = acc;
-}
-
-template <class T, int FIN>
-__global__ __launch_bounds__(kSweepWgThreads) void k_tri_wg(
-    const int32_t *__restrict__ lptr, int32_t nlev, const int4 *__restrict__ rec,
-    const int32_t *__restrict__ dcol, const T *__restrict__ dcoef, const T *__restrict__ sc,
-    const T *__restrict__ in, T *out) {
-  for (int32_t L = 0; L < nlev; L++) {
-    const int32_t k1 = lptr[L + 1];
-    for (int32_t k = lptr[L] + (int32_t)threadIdx.x; k < k1; k += kSweepWgThreads)
-      tri_row<T, FIN>(rec[k], dcol, dcoef, sc[k], in, out);
-    __syncthreads();  // the level's rows are written before the next reads them
-  }
-}
-
-// The pipelined form (levels at most kSweepWgThreads rows wide, one row per
-// thread and level): while level L runs, the dependency entries of level
-// L+1 and the row records of level L+2 are already in flight, and the
-// values of the last kTriRing level-order positions live in LDS (dpos >= 0
-// names the slot; older values are read from out), so a level costs LDS
-// reads, a store and the barrier.  Within a wave that has rows the prefetch
-// loads are unconditional (clamped to entry 0 for missing rows), waves
-// without rows load nothing, and the level loop is unrolled six times so
-// that no register of a load in flight is ever copied: together these keep
-// the compiler's wait counts exact, which is what lets the loads overlap.
-constexpr int kTriPre = 4;  // dependency entries held in registers per row
-
-template <class T> struct TriHead {
-  int32_t i, d0, d1;  // d1 < 0: no row
-  T s, init;
-};
-template <class T> struct TriDeps {
-  int32_t c[kTriPre], p[kTriPre];
-  T a[kTriPre];
-};
-
-template <class T, int FIN>
-__device__ __forceinline__ void tri_head(TriHead<T> &h, bool valid, int32_t k,
-                                         const int4 *__restrict__ rec, const T *__restrict__ sc,
-                                         const T *__restrict__ in, const T *out) {
-  const int32_t kk = valid ? k : 0;
-  const int4 r = rec[kk];
-  h.i = r.x;
-  h.d0 = r.y;
-  h.d1 = valid ? r.z : -1;
-  h.s = sc[kk];
-  h.init = FIN == 1 ? out[r.x] : in[r.x];
-}
-
-template <class T>
-__device__ __forceinline__ void tri_deps(const TriHead<T> &h, TriDeps<T> &d,
-                                         const int32_t *__restrict__ dcol,
-                                         const int32_t *__restrict__ dpos,
-                                         const T *__restrict__ dcoef) {
-#pragma unroll
-  for (int u = 0; u < kTriPre; u++) {
-    const int32_t e = h.d0 + u < h.d1 ? h.d0 + u : 0;
-    d.c[u] = dcol[e];
-    d.p[u] = dpos[e];
-    d.a[u] = dcoef[e];
-  }
-}
-
-// the values read by row h: the first kTriPre from the prefetched entries,
-// then the product sum over all of them in the row's order
-template <class T, int FIN>
-__device__ __forceinline__ void tri_finish(const TriHead<T> &h, const TriDeps<T> &d, int32_t k,
-                                           const T *zv, T *ring,
-                                           const int32_t *__restrict__ dcol,
-                                           const int32_t *__restrict__ dpos,
-                                           const T *__restrict__ dcoef, T *out) {
-  using Acc = typename std::conditional<FIN == 1, double, T>::type;
-  Acc acc = FIN == 1 ? (Acc)0 : (Acc)h.init;
-#pragma unroll
-  for (int u = 0; u < kTriPre; u++) {
-    if (h.d0 + u < h.d1) {
-      const T p = d.a[u] * zv[u];
-      if (FIN == 1)
-        acc = acc + (double)p;
-      else
-        acc = acc - p;
-    }
-  }
-  for (int32_t e = h.d0 + kTriPre; e < h.d1; e += kTriChunk) {
-    int32_t c[kTriChunk], q[kTriChunk];
-    T a[kTriChunk], z[kTriChunk];
-#pragma unroll
-    for (int u = 0; u < kTriChunk; u++) {
-      const bool v = e + u < h.d1;
-      c[u] = v ? dcol[e + u] : 0;
-      q[u] = v ? dpos[e + u] : 0;
-      a[u] = v ? dcoef[e + u] : (T)0;
-    }
-#pragma unroll
-    for (int u = 0; u < kTriChunk; u++)
-      z[u] = e + u < h.d1 ? (q[u] >= 0 ? ring[q[u] & (kTriRing - 1)] : out[c[u]]) : (T)0;
-#pragma unroll
-    for (int u = 0; u < kTriChunk; u++) {
-      if (e + u < h.d1) {
-        const T p = a[u] * z[u];
-        if (FIN == 1)
-          acc = acc + (double)p;
-        else
-          acc = acc - p;
-      }
-    }
-  }
-  T v;
-  if (FIN == 0)
-    v = acc * h.s;
-  else if (FIN == 1)
-    v = (T)((double)h.init - acc * (double)h.s);
-  else if (FIN == 2)
-    v = acc / h.s;
-  else
-    v = acc;
-  out[h.i] = v;
-  ring[k & (kTriRing - 1)] = v;
-}
-
-template <class T, int FIN>
-__global__ __launch_bounds__(kSweepWgThreads) void k_tri_pipe(
-    const int32_t *__restrict__ lptr, int32_t nlev, const int4 *__restrict__ rec,
-    const int32_t *__restrict__ dcol, const int32_t *__restrict__ dpos,
-    const T *__restrict__ dcoef, const T *__restrict__ sc, const T *__restrict__ in, T *out) {
-  __shared__ T ring[kTriRing];
-  const int32_t t = (int32_t)threadIdx.x;
-  // level L covers positions [lptr[L], lptr[L+1]); kb[] holds the bounds of
-  // levels L, L+1 and L+2 as the loop advances
-  int32_t k0 = lptr[0], k1 = nlev > 0 ? lptr[1] : 0, k2 = nlev > 1 ? lptr[2] : k1;
-  TriHead<T> h0, h1, h2;
-  TriDeps<T> e0, e1;
-  tri_head<T, FIN>(h0, k0 + t < k1, k0 + t, rec, sc, in, out);
-  tri_deps(h0, e0, dcol, dpos, dcoef);
-  tri_head<T, FIN>(h1, nlev > 1 && k1 + t < k2, k1 + t, rec, sc, in, out);
-  h2.d1 = -1;
-  // one level: cur (its entries cd) runs, the entries of nxt and the record
-  // of the level after it (into nn) are loaded
-  const int32_t w0 = t & ~63;  // first thread of this wave: waves without rows load nothing
-  auto step = [&](int32_t L, TriHead<T> &cur, TriDeps<T> &cd, TriHead<T> &nxt, TriDeps<T> &nd,
-                  TriHead<T> &nn) {
-    const int32_t k3 = L + 3 <= nlev ? lptr[L + 3] : k2;
-    T zv[kTriPre];
-#pragma unroll
-    for (int u = 0; u < kTriPre; u++)
-      zv[u] = cur.d0 + u < cur.d1
-                  ? (cd.p[u] >= 0 ? ring[cd.p[u] & (kTriRing - 1)] : out[cd.c[u]])
-                  : (T)0;
-    // the values (and every load of the step before) have arrived before the
-    // prefetch loads go out, so nothing below waits for those
-    __builtin_amdgcn_s_waitcnt(0);
-    if (w0 < k2 - k1) tri_deps(nxt, nd, dcol, dpos, dcoef);
-    if (L + 2 < nlev && w0 < k3 - k2)
-      tri_head<T, FIN>(nn, k2 + t < k3, k2 + t, rec, sc, in, out);
-    else
-      nn.d1 = -1;
-    if (cur.d1 >= 0) tri_finish<T, FIN>(cur, cd, k0 + t, zv, ring, dcol, dpos, dcoef, out);
-    __syncthreads();  // the level's values (LDS and out) are written before the next reads them
-    k0 = k1;
-    k1 = k2;
-    k2 = k3;
-  };
-  for (int32_t L = 0; L < nlev; L += 6) {
-    step(L, h0, e0, h1, e1, h2);
-    if (L + 1 >= nlev) break;
-    step(L + 1, h1, e1, h2, e0, h0);
-    if (L + 2 >= nlev) break;
-    step(L + 2, h2, e0, h0, e1, h1);
-    if (L + 3 >= nlev) break;
-    step(L + 3, h0, e1, h1, e0, h2);
-    if (L + 4 >= nlev) break;
-    step(L + 4, h1, e0, h2, e1, h0);
-    if (L + 5 >= nlev) break;
-    step(L + 5, h2, e1, h0, e0, h1);
-  }
-}
-
-// The staged form: levels are grouped into blocks of at most kStPos rows
-// and kStDeps dependency entries (whole levels, contiguous in the plan).
-// While the rows of block b run out of LDS, the records of block b+1 are
-// loaded into registers by the whole workgroup in one coalesced pass and
-// written to the other LDS buffer afterwards, so a level costs only LDS
-// traffic, its stores and the barrier; global memory latency is paid once
-// per block.  The initial values (in, or out for the SOR backward sweep)
-// are gathered into level order by k_tri_gather before the sweep.
-constexpr int kStPos = 1024, kStDeps = 1536;
-
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_tri_gather(int64_t n, const int4 *__restrict__ rec,
-                                                       const T *__restrict__ src, T *dst) {
-  const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (k < n) dst[k] = src[rec[k].x];
-}
-
-template <class T, int FIN>
-__global__ __launch_bounds__(kSweepWgThreads) void k_tri_staged(
-    const int4 *__restrict__ blk, int32_t nblk, const int32_t *__restrict__ lptr,
-    const int4 *__restrict__ rec, const T *__restrict__ sc, const T *__restrict__ ginit,
-    const int32_t *__restrict__ dpos, const int32_t *__restrict__ dcol,
-    const T *__restrict__ dcoef, T *out) {
-  __shared__ int4 s_rec[2][kStPos];
-  __shared__ T s_sc[2][kStPos], s_init[2][kStPos];
-  __shared__ int32_t s_dpos[2][kStDeps], s_dcol[2][kStDeps];
-  __shared__ T s_coef[2][kStDeps];
-  __shared__ int32_t s_lptr[2][kStPos];
-  __shared__ T ring[kTriRing];
-  constexpr int kDU = (kStDeps + kSweepWgThreads - 1) / kSweepWgThreads;
-  const int32_t t = (int32_t)threadIdx.x;
-  // registers of the block being loaded (block descriptors: x = first
-  // level, y = first position, z = first dependency entry)
-  int4 g_rec;
-  T g_sc, g_init, g_coef[kDU];
-  int32_t g_dpos[kDU], g_dcol[kDU], g_lptr;
-  auto load = [&](const int4 B0, const int4 B1) {
-    const int32_t np = B1.y - B0.y, nd = B1.z - B0.z, nl = B1.x - B0.x;
-    const int32_t kp = B0.y + (t < np ? t : 0);
-    g_rec = rec[kp];
-    g_sc = sc[kp];
-    g_init = ginit[kp];
-#pragma unroll
-    for (int u = 0; u < kDU; u++) {
-      const int32_t dd = t + u * kSweepWgThreads;
-      const int32_t idx = dd < nd ? B0.z + dd : 0;
-      g_dpos[u] = dpos[idx];
-      g_dcol[u] = dcol[idx];
-      g_coef[u] = dcoef[idx];
-    }
-    g_lptr = lptr[B0.x + (t < nl ? t : 0)];
-  };
-  auto store = [&](int buf, const int4 B0, const int4 B1) {
-    const int32_t np = B1.y - B0.y, nd = B1.z - B0.z, nl = B1.x - B0.x;
-    if (t < np) {
-      s_rec[buf][t] = g_rec;
-      s_sc[buf][t] = g_sc;
-      s_init[buf][t] = g_init;
-    }
-#pragma unroll
-    for (int u = 0; u < kDU; u++) {
-      const int32_t dd = t + u * kSweepWgThreads;
-      if (dd < nd && dd < kStDeps) {
-        s_dpos[buf][dd] = g_dpos[u];
-        s_dcol[buf][dd] = g_dcol[u];
-        s_coef[buf][dd] = g_coef[u];
-      }
-    }
-    if (t < nl) s_lptr[buf][t] = g_lptr;
-  };
-  int4 B0 = blk[0], B1 = blk[1];
-  load(B0, B1);
-  store(0, B0, B1);
-  __syncthreads();
-  for (int32_t b = 0; b < nblk; b++) {
-    const int buf = b & 1;
-    const int4 N0 = B1, N1 = b + 2 <= nblk ? blk[b + 2] : B1;
-    if (b + 1 < nblk) load(N0, N1);  // in flight while this block runs
-    const int32_t nl = B1.x - B0.x;
-    for (int32_t l = 0; l < nl; l++) {
-      const int32_t ka = s_lptr[buf][l], kb = l + 1 < nl ? s_lptr[buf][l + 1] : B1.y;
-      if (ka + t < kb) {
-        const int32_t kk = ka + t - B0.y;
-        const int4 rc = s_rec[buf][kk];
-        const int32_t d0 = rc.y - B0.z, d1 = rc.z - B0.z;
-        using Acc = typename std::conditional<FIN == 1, double, T>::type;
-        const T init = s_init[buf][kk];
-        Acc acc = FIN == 1 ? (Acc)0 : (Acc)init;
-        for (int32_t d = d0; d < d1; d++) {
-          const int32_t q = s_dpos[buf][d];
-          const T z = q >= 0 ? ring[q & (kTriRing - 1)] : out[s_dcol[buf][d]];
-          const T p = s_coef[buf][d] * z;
-          if (FIN == 1)
-            acc = acc + (double)p;
-          else
-            acc = acc - p;
-        }
-        const T s = s_sc[buf][kk];
-        T v;
-        if (FIN == 0)
-          v = acc * s;
-        else if (FIN == 1)
-          v = (T)((double)init - acc * (double)s);
-        else if (FIN == 2)
-          v = acc / s;
-        else
-          v = acc;
-        out[rc.x] = v;
-        ring[(ka + t) & (kTriRing - 1)] = v;
-      }
-      __syncthreads();  // the level's values are written before the next reads them
-    }
-    if (b + 1 < nblk) store(buf ^ 1, N0, N1);
-    __syncthreads();
-    B0 = N0;
-    B1 = N1;
-  }
-}
-
-// The dependency-driven form, for plans too large or too wide for one
-// workgroup: persistent waves take 64 consecutive level-order positions at a
-// time from a ticket counter and each lane computes its row as soon as the
-// rows it reads are written, with no barrier between levels.  Readiness
-// travels with the value: before the sweep every out_i holds kEmpty, a
-// signalling NaN that no arithmetic produces, and a row publishes its value
-// with one device-coherent atomic exchange, so a reader that finds
-// something else has the final value.  A lane loads its entries eight at a
-// time (plain loads) and consumes them strictly in the row's order; at the
-// first one still kEmpty it polls that one entry with a device-coherent
-// atomic read (a plain load may keep seeing a cached copy) until it is
-// written, then goes on, so the arithmetic is the serial sweep's.  Rows only read rows of earlier
-// levels, which sit at earlier positions, so their tickets were taken by
-// waves that are already running: the sweep cannot deadlock.  A lane that
-// has consumed none of its row's entries for kFlowSpinTicks of the 100 MHz
-// wall clock gives up: it publishes NaN and raises the plan's stall flag
-// (ticket[1]), so the kernel always ends and the solver returns
-// MGX_ERR_TIMEOUT.  At most 1024 waves x 64 rows are in flight, so a valid
-// plan's longest wait is 65536 dependency hops (measured 4-7 us each), far
-// inside the 2 s limit.
-constexpr int kFlowThreads = 256;
-constexpr int kFlowBlocks = 256;
-constexpr uint64_t kFlowSpinTicks = 200000000;  // 2 s without progress
-// plans whose levels hold kFlowMinWidth rows on average take the
-// dependency-driven form when they have at least kFlowMinRows rows or a
-// level wider than one workgroup's block; deep plans (a long chain beside
-// wide levels) stay in one workgroup, which sweeps any width level by level
+constexpr int kChWaves = 4;      // one per SIMD
+constexpr int kRing = 1024;      // values of earlier chunks that a wave keeps
+// Rows of a wave.  Narrow levels (2D grids): long ranges, so that the chain
+// crosses few chunks.  Levels of kWideLevel rows on average or more (3D
+// grids): short ranges, so that a level's rows spread over the chip.  Per
+// SOR-PCG iteration, FP64, with 2048 / 1024 / 256 rows: 2D 5-point 256^2
+// (128 rows a level) 0.37 / 0.40 / 0.42 ms, 1000^2 (500) 1.46 / 1.43 / 2.57
+// ms; 3D 27-point 96^3 (1328) 2.06 / 1.87 / 1.68 ms, 128^3 (2356) 2.86 /
+// 2.58 / 2.36 ms, 7-point 100^3 (3356) 0.95 / 0.82 / 0.77 ms.
+constexpr int kWaveRows = 2048, kWaveRowsWide = 256, kWideLevel = 1000;
+// Scattered matrices: a chunk of 8192 rows reads more than kScattered
+// distinct values of earlier chunks per row and wave (grids: up to 1.3).  The
+// dependency-driven form takes them when their levels can fill the chip (at
+// least kFlowMinRows rows, kFlowMinWidth a level): 300000-row random
+// M-matrix, 5085 rows a level, 0.65 ms an iteration against 1.77 ms in
+// chunks.  Smaller ones run in chunks of kWaveRowsScattered rows a wave:
+// 20000 rows, 0.69 ms.
+constexpr double kScattered = 3.0;
+constexpr int kWaveRowsScattered = 64;
 constexpr int64_t kFlowMinRows = 1 << 17, kFlowMinWidth = 256;
+constexpr uint64_t kSpinTicks = 200000000;  // 2 s of the 100 MHz clock without progress
 
-template <class T> struct FlowBits;
-template <> struct FlowBits<double> {
+// batch header: x, y = lanes whose row starts a level, z = rows | values of
+// earlier chunks << 8 | kPart... (a batch with part of its rows' entries:
+// one level, the sums go on in the next batch or come from the last)
+constexpr uint32_t kPartFirst = 1u << 20, kPartMid = 1u << 21, kPartLast = 1u << 22;
+// LDS slots: the chunk's crows values, the waves' rings, one slot that
+// holds 0; then the ticket
+constexpr uint32_t slot_zero(uint32_t crows) { return crows + kChWaves * kRing; }
+static_assert(slot_zero(kChWaves * kWaveRows) < 65536, "slots are stored in 16 bits");
+
+template <class T> struct SweepBits;
+template <> struct SweepBits<double> {
   using U = uint64_t;
   static constexpr U kEmpty = 0x7ff0deadbeef0001ull, kNan = 0x7ff8000000000000ull;
 };
-template <> struct FlowBits<float> {
+template <> struct SweepBits<float> {
   using U = uint32_t;
   static constexpr U kEmpty = 0x7f80dea1u, kNan = 0x7fc00000u;
 };
 
-// ginit[k] = the initial value of row rec[k].x (out for the SOR backward
-// sweep, in otherwise), then out of that row = kEmpty; in may alias out
+template <class T> struct TriArgs {
+  int64_t n;
+  int32_t crows, nchunk, rev;  // rows per chunk, chunks, sweep from the last row
+  const int64_t *wave;
+  const int4 *hdr;
+  const int32_t *row, *ext;
+  const uint16_t *slot;
+  const T *coef, *isc;
+  T *out;
+  uint32_t *ticket;
+};
+
+// isc[2k] = the initial value of row[k] (out for the SOR backward sweep, in
+// otherwise), then out of that row = kEmpty, a signalling NaN that no
+// arithmetic produces; in may alias out
 template <class T, int FIN>
-__global__ __launch_bounds__(kBlock) void k_flow_init(int64_t n, const int4 *__restrict__ rec,
-                                                      const T *in, T *out, T *ginit,
-                                                      uint32_t *ticket) {
-  using U = typename FlowBits<T>::U;
+__global__ __launch_bounds__(kBlock) void k_tri_init(int64_t n, const int32_t *__restrict__ row,
+                                                     const T *in, T *out, T *isc,
+                                                     uint32_t *ticket) {
+  using U = typename SweepBits<T>::U;
   const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (k == 0) *ticket = 0u;
   if (k < n) {
-    const int32_t i = rec[k].x;
-    ginit[k] = FIN == 1 ? out[i] : in[i];
-    reinterpret_cast<U *>(out)[i] = FlowBits<T>::kEmpty;
+    const int32_t i = row[k];
+    isc[2 * k] = FIN == 1 ? out[i] : in[i];
+    reinterpret_cast<U *>(out)[i] = SweepBits<T>::kEmpty;
   }
 }
+
+// A wave waiting for values: true when nothing in the whole sweep has
+// progressed for kSpinTicks (ticket[2] counts steps done, in groups); the
+// wave then gives up (its rows become NaN) and ticket[1] makes the solver
+// return MGX_ERR_TIMEOUT, so every wait ends.
+struct SpinWatch {
+  uint64_t t0 = 0;
+  uint32_t seen = 0, spins = 0;
+  __device__ __forceinline__ bool give_up(uint32_t *ticket) {
+    if (__builtin_expect((++spins & 255u) != 0, 1)) return false;
+    const uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane(
+        (int)__hip_atomic_load(ticket + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    const uint64_t now = wall_clock64();
+    if (spins == 256u || p != seen) {
+      seen = p;
+      t0 = now;
+      return false;
+    }
+    if (now - t0 <= kSpinTicks &&
+        __hip_atomic_load(ticket + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+      return false;
+    __hip_atomic_store(ticket + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+  }
+};
+
+// plan data at a uniform address, by scalar loads: they don't queue behind
+// the vector loads in flight
+template <class V> __device__ __forceinline__ V scalar_get(const void *p, int64_t i) {
+  typedef const __attribute__((address_space(4))) V CV;
+  return ((CV *)p)[i];
+}
+
+// Entries per row and batch D (even): batches loaded ahead, registers of 64
+// values of earlier chunks per batch, slots stored per lane and load
+template <int D> struct Width {
+  static constexpr int kAhead = D <= 4 ? 4 : 3, kFar = D <= 4 ? 1 : 3;
+  static constexpr int kSlotLoad = D < 8 ? D : 8, kSlotLoads = (D + kSlotLoad - 1) / kSlotLoad;
+  static constexpr int kSlots = kSlotLoad * kSlotLoads;
+};
+
+// one batch's data, in registers from kAhead batches before it runs
+template <class T, int D> struct BatchRegs {
+  T coef[D], init, sc;
+  uint32_t slot[Width<D>::kSlots / 2];
+  int32_t row, col[Width<D>::kFar];
+  typename SweepBits<T>::U ext[Width<D>::kFar];
+};
+
+// FIN 0: out = acc * sc (SOR forward); 1: SOR backward, acc in double from
+// 0, out = (T)((double)out - acc * (double)sc); 2: out = acc / sc; 3: out = acc
+template <class T, int FIN, int D>
+__global__ __launch_bounds__(64 * kChWaves) void k_tri_chunk(const TriArgs<T> a) {
+  using U = typename SweepBits<T>::U;
+  using Acc = typename std::conditional<FIN == 1, double, T>::type;
+  using W = Width<D>;
+  typedef int32_t I4 __attribute__((ext_vector_type(4)));
+  typedef T V2 __attribute__((ext_vector_type(2)));
+  typedef uint32_t SV __attribute__((ext_vector_type(W::kSlotLoad < 4 ? 2 : W::kSlotLoad / 2)));
+  constexpr U kEmpty = SweepBits<T>::kEmpty;
+  constexpr int P = W::kAhead, X = W::kFar, SL = W::kSlotLoad;
+  extern __shared__ __align__(16) unsigned char tri_lds[];
+  U *const s_val = reinterpret_cast<U *>(tri_lds);
+  const uint32_t zero = slot_zero((uint32_t)a.crows);
+  uint32_t *const s_ticket = reinterpret_cast<uint32_t *>(s_val + zero + 1);
+  const uint32_t lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  U *const ob = reinterpret_cast<U *>(a.out);
+  U *const ring = s_val + a.crows + w * kRing;
+  auto lds_at = [&](uint32_t byte) -> U * { return reinterpret_cast<U *>(tri_lds + byte); };
+  auto lds_get = [&](uint32_t byte) -> U {
+    return __hip_atomic_load(lds_at(byte), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  auto far_get = [&](int32_t row) -> U {
+    return __hip_atomic_load(ob + row, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  if (threadIdx.x == 0) s_val[zero] = (U)0;
+  for (;;) {
+    if (threadIdx.x == 0)
+      *s_ticket =
+          __hip_atomic_fetch_add(a.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = (int)threadIdx.x; i < a.crows; i += 64 * kChWaves) s_val[i] = kEmpty;
+    __syncthreads();
+    const int32_t ch = __builtin_amdgcn_readfirstlane((int)*s_ticket);
+    if (ch >= a.nchunk) break;
+    // LDS slot of row i: its sweep position (i, or n - 1 - i) less the
+    // chunk's first, as (i ^ flip) + off
+    const uint32_t flip = a.rev ? ~0u : 0u;
+    const uint32_t off = (a.rev ? (uint32_t)a.n : 0u) - (uint32_t)(ch * a.crows);
+    const int64_t *const wv = a.wave + ((int64_t)ch * kChWaves + w) * 4;
+    const int64_t s0 = scalar_get<int64_t>(wv, 0), s1 = scalar_get<int64_t>(wv, 4);
+    int64_t le = scalar_get<int64_t>(wv, 1), lr = scalar_get<int64_t>(wv, 2),
+            lx = scalar_get<int64_t>(wv, 3);
+    uint32_t xpos = 0;  // values of earlier chunks taken so far
+    BatchRegs<T, D> R[P];
+    I4 h[P];
+    auto load = [&](BatchRegs<T, D> &r, const I4 hd) {
+      const uint32_t m = hd.z & 127u;
+      // le counts rows: D coefficients (pairs of all rows, then the next
+      // pairs) and kSlots slots each
+      const V2 *cp = reinterpret_cast<const V2 *>(a.coef + le * D);
+#pragma unroll
+      for (int u = 0; u < D; u += 2, cp += m) {
+        const V2 c2 = cp[lane];
+        r.coef[u] = c2[0];
+        r.coef[u + 1] = c2[1];
+      }
+      const uint32_t *sp = reinterpret_cast<const uint32_t *>(a.slot + le * W::kSlots);
+#pragma unroll
+      for (int g = 0; g < W::kSlotLoads; g++, sp += m * (SL / 2)) {
+        if constexpr (SL == 2) {
+          r.slot[g] = sp[lane];
+        } else {
+          const SV sv = reinterpret_cast<const SV *>(sp)[lane];
+#pragma unroll
+          for (int q = 0; q < SL / 2; q++) r.slot[g * (SL / 2) + q] = sv[q];
+        }
+      }
+      const V2 is = reinterpret_cast<const V2 *>(a.isc + 2 * lr)[lane];
+      r.init = is[0];
+      r.sc = is[1];
+      r.row = (a.row + lr)[lane];
+#pragma unroll
+      for (int q = 0; q < X; q++) r.col[q] = (a.ext + lx + 64 * q)[lane];
+      le += m;
+      lr += (hd.z & kPartLast) || !(hd.z & (kPartFirst | kPartLast | kPartMid)) ? m : 0u;
+      lx += (hd.z >> 8) & 1023u;
+    };
+    auto far_load = [&](BatchRegs<T, D> &r, const I4 hd) {
+      if ((hd.z >> 8) & 1023u) {
+#pragma unroll
+        for (int q = 0; q < X; q++) r.ext[q] = far_get(r.col[q]);
+      }
+    };
+    if (s0 < s1) {
+#pragma unroll
+      for (int k = 0; k < P; k++) {
+        h[k] = scalar_get<I4>(a.hdr, s0 + k);
+        load(R[k], h[k]);
+      }
+      far_load(R[0], h[0]);
+    }
+    Acc carry = (Acc)0;
+    for (int64_t s = s0; s < s1; s += P) {
+#pragma unroll
+      for (int k = 0; k < P; k++) {
+        BatchRegs<T, D> &r = R[k];
+        BatchRegs<T, D> &rn = R[(k + 1) % P];
+        const I4 hd = h[k];
+        const I4 hn = scalar_get<I4>(a.hdr, s + P + k);
+        far_load(rn, h[(k + 1) % P]);
+        const uint32_t m = hd.z & 127u, ne = (hd.z >> 8) & 1023u;
+        // values that are not there yet go into the ring as the marker
+        auto take = [&]() {
+#pragma unroll
+          for (int q = 0; q < X; q++)
+            if (64 * q + lane < ne) ring[(xpos + 64 * q + lane) & (kRing - 1)] = r.ext[q];
+          asm volatile("" ::: "memory");
+        };
+        if (ne) take();
+        if (ne && m == 0) {
+          // (no row of this batch will look again: wait here)
+          SpinWatch sw;
+          for (;;) {
+            bool miss = false;
+#pragma unroll
+            for (int q = 0; q < X; q++) miss = miss || (64 * q + lane < ne && r.ext[q] == kEmpty);
+            if (!__any(miss) || sw.give_up(a.ticket)) break;
+#pragma unroll
+            for (int q = 0; q < X; q++) r.ext[q] = far_get(r.col[q]);
+          }
+          take();
+        }
+        // the level of the lane's row in this batch, its values' and its own
+        // place in LDS
+        const uint64_t starts = (uint64_t)(uint32_t)hd.y << 32 | (uint32_t)hd.x;
+        const int levels = __popcll(starts);
+        int my = (int)__builtin_amdgcn_mbcnt_hi(
+            (uint32_t)hd.y, __builtin_amdgcn_mbcnt_lo((uint32_t)hd.x, 0u));
+        my += (int)((starts >> lane) & 1u) - 1;
+        if (lane >= m) my = -1;
+        uint32_t from[D];
+#pragma unroll
+        for (int u = 0; u < D; u++)
+          from[u] = (u & 1 ? r.slot[u / 2] >> 16 : r.slot[u / 2] & 0xffffu) * (uint32_t)sizeof(U);
+        U *const to = lds_at((((uint32_t)r.row ^ flip) + off) * (uint32_t)sizeof(U));
+        U *const out = ob + r.row;
+        const bool part = (hd.z & (kPartFirst | kPartMid | kPartLast)) != 0;
+        Acc begin = FIN == 1 ? (Acc)0 : (Acc)r.init;
+        if (part && !(hd.z & kPartFirst)) begin = carry;
+        const bool last = !part || (hd.z & kPartLast);
+        for (int j = 0; j < levels; j++) {
+          Acc acc = begin;
+          U z[D];
+          auto sum = [&]() {
+#pragma unroll
+            for (int u = 0; u < D; u++) z[u] = lds_get(from[u]);
+            acc = begin;
+#pragma unroll
+            for (int u = 0; u < D; u++) {
+              const T p = r.coef[u] * __builtin_bit_cast(T, z[u]);
+              if (FIN == 1)
+                acc = acc + (double)p;
+              else
+                acc = acc - p;
+            }
+          };
+          bool odd = false;
+          if (my == j) {
+            sum();
+            odd = acc != acc;
+          }
+          if (__builtin_expect(__any(odd), 0)) {
+            // a value that another wave of the chunk has not written yet, or
+            // that an earlier chunk had not when it was asked for; or a NaN
+            SpinWatch sw;
+            for (;;) {
+              if (ne) {
+#pragma unroll
+                for (int q = 0; q < X; q++) r.ext[q] = far_get(r.col[q]);
+                take();
+              }
+              bool miss = false;
+              if (my == j) {
+                sum();
+#pragma unroll
+                for (int u = 0; u < D; u++) miss = miss || z[u] == kEmpty;
+              }
+              if (!__any(miss) || sw.give_up(a.ticket)) break;  // (the marker: a NaN row)
+            }
+          }
+          if (my == j) {
+            if (last) {
+              T v;
+              if (FIN == 0)
+                v = acc * r.sc;
+              else if (FIN == 1)
+                v = (T)((double)r.init - acc * (double)r.sc);
+              else if (FIN == 2)
+                v = acc / r.sc;
+              else
+                v = acc;
+              const U vb = __builtin_bit_cast(U, v);
+              __hip_atomic_store(to, vb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              __hip_atomic_store(out, vb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else {
+              carry = acc;
+            }
+          }
+          asm volatile("" ::: "memory");  // the wave's next level reads these values
+        }
+        xpos += ne;
+        h[k] = hn;
+        load(r, hn);
+      }
+      if (lane == 0)
+        __hip_atomic_fetch_add(a.ticket + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();  // the chunk's values are cleared next
+  }
+}
+
+// The dependency-driven form, for matrices whose rows read scattered rows
+// all over the matrix (kScattered): hardly any dependency stays inside a
+// chunk there, and what bounds the sweep is the number of values fetched.
+// Persistent waves take 64 consecutive level-order positions at a time from
+// a ticket counter and each lane computes its row as soon as the rows it
+// reads are written.  A lane loads its entries eight at a time (plain loads)
+// and consumes them strictly in the row's order; at the first one still
+// kEmpty it polls that one entry with a device-coherent atomic read (a plain
+// load may keep seeing a cached copy) until it is written, then goes on, so
+// the arithmetic is the serial sweep's.  Rows only read rows of earlier
+// levels, which sit at earlier positions, so their tickets were taken by
+// waves that are already running: the sweep cannot deadlock.  A lane that
+// has consumed none of its row's entries for kSpinTicks gives up: it
+// publishes NaN and raises the plan's stall flag (ticket[1]), so the kernel
+// always ends and the solver returns MGX_ERR_TIMEOUT.  At most 1024 waves x
+// 64 rows are in flight, so a valid plan's longest wait is 65536 dependency
+// hops (measured 4-7 us each), far inside the 2 s limit.
+constexpr int kFlowThreads = 256;
+constexpr int kFlowBlocks = 256;
+constexpr int kTriChunk = 8;
 
 template <class T, int FIN>
 __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
     int32_t n, const int4 *__restrict__ rec, const int32_t *__restrict__ dcol,
-    const T *__restrict__ dcoef, const T *__restrict__ sc, const T *__restrict__ ginit, T *out,
-    uint32_t *ticket) {
-  using U = typename FlowBits<T>::U;
+    const T *__restrict__ dcoef, const T *__restrict__ isc, T *out, uint32_t *ticket) {
+  using U = typename SweepBits<T>::U;
   using Acc = typename std::conditional<FIN == 1, double, T>::type;
   U *ob = reinterpret_cast<U *>(out);
   const int lane = (int)(threadIdx.x & 63);
@@ -440,7 +418,7 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
     const int4 rc = has ? rec[k] : make_int4(0, 0, 0, 0);
     int32_t d = rc.y;
     const int32_t d1 = has ? rc.z : rc.y;
-    const T init = has ? ginit[k] : (T)0;
+    const T init = has ? isc[2 * (int64_t)k] : (T)0;
     Acc acc = FIN == 1 ? (Acc)0 : (Acc)init;
     uint64_t t0 = wall_clock64();  // the lane's last progress
     int32_t wc = -1;  // >= 0: column of entry d, which was still kEmpty
@@ -453,7 +431,7 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
         if (wc >= 0) {
           const U z = __hip_atomic_fetch_or(ob + wc, (U)0, __ATOMIC_RELAXED,
                                             __HIP_MEMORY_SCOPE_AGENT);
-          if (z != FlowBits<T>::kEmpty) {
+          if (z != SweepBits<T>::kEmpty) {
             const T p = wa * __builtin_bit_cast(T, z);
             if (FIN == 1)
               acc = acc + (double)p;
@@ -484,7 +462,7 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
 #pragma unroll
           for (int u = 0; u < kTriChunk; u++) {
             if (!stop && d + u < d1) {
-              if (zb[u] == FlowBits<T>::kEmpty) {
+              if (zb[u] == SweepBits<T>::kEmpty) {
                 stop = true;
                 wc = c[u];
                 wa = a[u];
@@ -501,14 +479,14 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
           d += taken;
           if (taken > 0) t0 = wall_clock64();
         }
-        if (d < d1 && wc >= 0 && wall_clock64() - t0 > kFlowSpinTicks) {
-          acc = (Acc)__builtin_bit_cast(T, FlowBits<T>::kNan);
+        if (d < d1 && wc >= 0 && wall_clock64() - t0 > kSpinTicks) {
+          acc = (Acc)__builtin_bit_cast(T, SweepBits<T>::kNan);
           d = d1;
           __hip_atomic_store(ticket + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
       }
       if (pending && d >= d1) {
-        const T s = sc[k];
+        const T s = isc[2 * (int64_t)k + 1];
         T v;
         if (FIN == 0)
           v = acc * s;
@@ -519,7 +497,7 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
         else
           v = acc;
         U vb = __builtin_bit_cast(U, v);
-        if (vb == FlowBits<T>::kEmpty) vb = FlowBits<T>::kNan;
+        if (vb == SweepBits<T>::kEmpty) vb = SweepBits<T>::kNan;
         __hip_atomic_exchange(ob + rc.x, vb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         pending = false;
       }
@@ -528,65 +506,110 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
   }
 }
 
-// coef[d] = vals[dent[d]]
+// coef[d] = vals[dent[d]], 0 where the plan has no entry
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_tri_pack(int64_t nd, const int32_t *__restrict__ dent,
                                                      const T *__restrict__ vals, T *coef) {
   const int64_t d = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (d < nd) coef[d] = vals[dent[d]];
+  if (d < nd) coef[d] = dent[d] < 0 ? (T)0 : vals[dent[d]];
 }
 
-// sc[k] = vec[pos ? pos[row_k] : row_k]
+// isc[2k + 1] = vec[pos ? pos[row[k]] : row[k]]
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_tri_scale(int64_t n, const int4 *__restrict__ rec,
+__global__ __launch_bounds__(kBlock) void k_tri_scale(int64_t n, const int32_t *__restrict__ row,
                                                       const T *__restrict__ vec,
-                                                      const int32_t *__restrict__ pos, T *sc) {
+                                                      const int32_t *__restrict__ pos, T *isc) {
   const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (k < n) {
-    const int32_t i = rec[k].x;
-    sc[k] = vec[pos ? pos[i] : i];
+    const int32_t i = row[k];
+    isc[2 * k + 1] = vec[pos ? pos[i] : i];
   }
+}
+
+template <class T>
+void tri_launch(Ctx *c, const TriPlan &P, void (*k)(TriArgs<T>), const TriArgs<T> &a) {
+  const size_t lds = (slot_zero((uint32_t)P.crows) + 1) * sizeof(T) + 16;
+  if (lds > 65536)
+    MGX_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  // small chunks: several workgroups share a compute unit
+  const unsigned grid = (unsigned)std::min(P.nchunk, 4 * c->num_cus);
+  k<<<grid, 64 * kChWaves, lds, c->stream>>>(a);
 }
 
 template <class T, int FIN>
-void tri_run_t(Ctx *c, const TriPlan &P, const T *coef, const T *sc, const T *in, T *out,
-               T *ginit) {
-  const SorLevels &L = P.lev;
-  if (L.nlev == 0) return;
+void tri_run_t(Ctx *c, const TriOp &op, const T *in, T *out) {
+  const TriPlan &P = *op.plan;
+  if (P.n == 0) return;
+  T *isc = static_cast<T *>(op.isc);
+  k_tri_init<T, FIN><<<(unsigned)((P.n + kBlock - 1) / kBlock), kBlock, 0, c->stream>>>(
+      P.n, P.d_row, in, out, isc, P.d_ticket);
   if (P.flow) {
-    const int64_t n = L.ptr[L.nlev];
-    k_flow_init<T, FIN><<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, c->stream>>>(
-        n, P.d_rec, in, out, ginit, P.d_ticket);
-    const int64_t want = (n + 63) / 64 / (kFlowThreads / 64) + 1;
+    const int64_t want = (P.n + 63) / 64 / (kFlowThreads / 64) + 1;
     k_tri_flow<T, FIN><<<(unsigned)std::min<int64_t>(want, kFlowBlocks), kFlowThreads, 0,
-                         c->stream>>>((int32_t)n, P.d_rec, P.d_dcol, coef, sc, ginit, out,
-                                      P.d_ticket);
-  } else if (P.nblk > 0) {
-    const int64_t n = L.ptr[L.nlev];
-    k_tri_gather<T><<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, c->stream>>>(
-        n, P.d_rec, FIN == 1 ? out : in, ginit);
-    k_tri_staged<T, FIN><<<1, kSweepWgThreads, 0, c->stream>>>(
-        P.d_blk, P.nblk, L.d_ptr, P.d_rec, sc, ginit, P.d_dpos, P.d_dcol, coef, out);
-  } else if (L.max_width <= kSweepWgThreads) {
-    k_tri_pipe<T, FIN><<<1, kSweepWgThreads, 0, c->stream>>>(
-        L.d_ptr, L.nlev, P.d_rec, P.d_dcol, P.d_dpos, coef, sc, in, out);
-  } else {
-    k_tri_wg<T, FIN><<<1, kSweepWgThreads, 0, c->stream>>>(L.d_ptr, L.nlev, P.d_rec, P.d_dcol,
-                                                           coef, sc, in, out);
+                         c->stream>>>((int32_t)P.n, P.d_rec, P.d_dcol,
+                                      static_cast<const T *>(op.coef), isc, out, P.d_ticket);
+    MGX_HIP(hipGetLastError());
+    return;
   }
+  const TriArgs<T> a{P.n,     P.crows, P.nchunk, P.rev,
+                     P.d_wave, P.d_hdr, P.d_row, P.d_ext, P.d_slot,
+                     static_cast<const T *>(op.coef), isc, out,
+                     P.d_ticket};
+  if (P.width == 2)
+    tri_launch(c, P, k_tri_chunk<T, FIN, 2>, a);
+  else if (P.width == 4)
+    tri_launch(c, P, k_tri_chunk<T, FIN, 4>, a);
+  else if (P.width == 8)
+    tri_launch(c, P, k_tri_chunk<T, FIN, 8>, a);
+  else
+    tri_launch(c, P, k_tri_chunk<T, FIN, 14>, a);
   MGX_HIP(hipGetLastError());
 }
 
 template <class T> void tri_run_fin(Ctx *c, const TriOp &op, const void *in, void *out) {
-  const T *coef = static_cast<const T *>(op.coef), *sc = static_cast<const T *>(op.sc);
   const T *x = static_cast<const T *>(in);
-  T *y = static_cast<T *>(out), *g = static_cast<T *>(op.ginit);
+  T *y = static_cast<T *>(out);
   switch (op.fin) {
-    case kTriMul: tri_run_t<T, 0>(c, *op.plan, coef, sc, x, y, g); break;
-    case kTriSorBack: tri_run_t<T, 1>(c, *op.plan, coef, sc, x, y, g); break;
-    case kTriDiv: tri_run_t<T, 2>(c, *op.plan, coef, sc, x, y, g); break;
-    default: tri_run_t<T, 3>(c, *op.plan, coef, sc, x, y, g); break;
+    case kTriMul: tri_run_t<T, 0>(c, op, x, y); break;
+    case kTriSorBack: tri_run_t<T, 1>(c, op, x, y); break;
+    case kTriDiv: tri_run_t<T, 2>(c, op, x, y); break;
+    default: tri_run_t<T, 3>(c, op, x, y); break;
   }
+}
+
+template <class V> V *upload(const std::vector<V> &h) {
+  V *d = (V *)dev_alloc(std::max<size_t>(h.size(), 1) * sizeof(V));
+  if (!h.empty()) MGX_HIP(hipMemcpy(d, h.data(), h.size() * sizeof(V), hipMemcpyHostToDevice));
+  return d;
+}
+
+template <class P, class V> V *upload_parts(const std::vector<P> &parts, std::vector<V> P::*m) {
+  size_t total = 0;
+  for (const P &p : parts) total += (p.*m).size();
+  V *d = (V *)dev_alloc(std::max<size_t>(total, 1) * sizeof(V));
+  size_t o = 0;
+  for (const P &p : parts) {
+    const std::vector<V> &h = p.*m;
+    if (!h.empty())
+      MGX_HIP(hipMemcpy(d + o, h.data(), h.size() * sizeof(V), hipMemcpyHostToDevice));
+    o += h.size();
+  }
+  return d;
+}
+
+struct WidthSizes {
+  int ahead, far, slot_load, slots;
+};
+template <int D> WidthSizes width_sizes() {
+  return {Width<D>::kAhead, Width<D>::kFar, Width<D>::kSlotLoad, Width<D>::kSlots};
+}
+
+// a batch without rows that takes the values of `rows`
+void push_values(std::vector<int4> &hdr, std::vector<int32_t> &ext,
+                 const std::vector<int32_t> &rows) {
+  hdr.push_back(make_int4(0, 0, (int32_t)((uint32_t)rows.size() << 8 | kPartMid), 0));
+  ext.insert(ext.end(), rows.begin(), rows.end());
 }
 
 bool dep_of(int filter, int64_t i, int32_t c) { return filter == 2 ? c > i : c < i; }
@@ -631,66 +654,242 @@ void build_tri_plan(const std::vector<int32_t> &ptr, const std::vector<int32_t> 
   L.nlev = nlev;
   L.max_width = 0;
   for (int32_t l = 0; l < nlev; l++) L.max_width = std::max(L.max_width, L.ptr[l + 1] - L.ptr[l]);
-  int64_t nd = 0;
-  for (int64_t i = 0; i < n; i++) nd += cnt[i];
-  std::vector<int4> rec(n);
-  std::vector<int32_t> dcol(std::max<int64_t>(nd, 1)), dent(std::max<int64_t>(nd, 1)),
-      dpos(std::max<int64_t>(nd, 1)), where(n);
-  for (int64_t k = 0; k < n; k++) where[rows[k]] = (int32_t)k;
-  int64_t d = 0;
-  for (int64_t k = 0; k < n; k++) {
-    const int32_t i = rows[k];
-    // a value read by this row is still in the LDS ring when no position of
-    // this row's level or an earlier one has overwritten its slot
-    const int64_t lo = (int64_t)L.ptr[lev[i] + 1] - kTriRing;
-    rec[k] = make_int4(i, (int32_t)d, (int32_t)(d + cnt[i]), 0);
-    for_deps(i, [&](int32_t j) {
-      dcol[d] = col[j];
-      dent[d] = ent ? (*ent)[j] : j;
-      dpos[d] = where[col[j]] >= lo ? where[col[j]] : -1;
-      d++;
-    });
+  P.n = n;
+  P.rev = filter == 2;
+  auto at = [&](int64_t i) { return P.rev ? n - 1 - i : i; };  // sweep position of row i
+  // scattered? (distinct values of earlier chunks in a sample of waves)
+  bool scattered = false;
+  {
+    const int64_t span = (int64_t)kChWaves * kWaveRows, nw = n / kWaveRows;
+    const int64_t step = std::max<int64_t>(1, nw / 32);
+    std::vector<int64_t> seen(nw > kChWaves ? n : 0, -1);
+    int64_t nrows = 0, far = 0;
+    for (int64_t v = kChWaves; v < nw; v += step) {
+      const int64_t base = v * kWaveRows / span * span;
+      for (int64_t p = v * kWaveRows; p < (v + 1) * kWaveRows; p++)
+        for_deps(at(p), [&](int32_t j) {
+          if (at(col[j]) < base && seen[col[j]] != v) seen[col[j]] = v, far++;
+        });
+      nrows += kWaveRows;
+    }
+    scattered = (double)far > kScattered * (double)nrows;
   }
-  P.ndeps = nd;
-  L.d_rows = (int32_t *)dev_alloc((size_t)std::max<int64_t>(n, 1) * 4);
-  L.d_ptr = (int32_t *)dev_alloc((size_t)(nlev + 1) * 4);
-  P.d_rec = (int4 *)dev_alloc((size_t)std::max<int64_t>(n, 1) * sizeof(int4));
-  P.d_dcol = (int32_t *)dev_alloc(dcol.size() * 4);
-  P.d_dent = (int32_t *)dev_alloc(dent.size() * 4);
-  P.d_dpos = (int32_t *)dev_alloc(dpos.size() * 4);
-  MGX_HIP(hipMemcpy(P.d_dpos, dpos.data(), dpos.size() * 4, hipMemcpyHostToDevice));
-  // large plans with wide levels sweep dependency-driven across the chip;
-  // the others in one workgroup, staged in blocks of whole levels when no
-  // level alone exceeds a block
-  P.flow = (L.max_width > kSweepWgRows || n >= kFlowMinRows) &&
-           n >= kFlowMinWidth * (int64_t)nlev;
+  P.d_ticket = (uint32_t *)dev_alloc(256);  // [0] ticket, [1] stall flag, [2] batches done
+  MGX_HIP(hipMemset(P.d_ticket, 0, 256));
+  L.d_rows = upload(rows);
+  L.d_ptr = upload(L.ptr);
+  P.flow = scattered && n >= kFlowMinRows && n >= kFlowMinWidth * (int64_t)nlev;
   if (P.flow) {
-    P.d_ticket = (uint32_t *)dev_alloc(256);
-    MGX_HIP(hipMemset(P.d_ticket, 0, 256));  // [0] ticket, [1] stall flag
+    int64_t nd = 0;
+    for (int64_t i = 0; i < n; i++) nd += cnt[i];
+    std::vector<int4> rec(n);
+    std::vector<int32_t> dcol(std::max<int64_t>(nd, 1)), dent(std::max<int64_t>(nd, 1));
+    int64_t d = 0;
+    for (int64_t k = 0; k < n; k++) {
+      const int32_t i = rows[k];
+      rec[k] = make_int4(i, (int32_t)d, (int32_t)(d + cnt[i]), 0);
+      for_deps(i, [&](int32_t j) {
+        dcol[d] = col[j];
+        dent[d++] = ent ? (*ent)[j] : j;
+      });
+    }
+    P.ndeps = nd;
+    P.nrow = n;
+    P.d_rec = upload(rec);
+    P.d_dcol = upload(dcol);
+    P.d_dent = upload(dent);
+    P.d_row = upload(rows);
+    P.built = true;
+    return;
   }
-  std::vector<int4> blk;
-  bool fits = !P.flow;
-  for (int32_t l = 0; l < nlev && fits; l++) {
-    const int32_t p0 = L.ptr[l], p1 = L.ptr[l + 1];
-    const int32_t e0 = rec[p0].y, e1 = rec[p1 - 1].z;
-    if (p1 - p0 > kStPos || e1 - e0 > kStDeps) fits = false;
-    if (blk.empty() || p1 - blk.back().y > kStPos || e1 - blk.back().z > kStDeps)
-      blk.push_back(make_int4(l, p0, e0, 0));
+  // rows of each wave in level order
+  const int64_t per = (n + kChWaves - 1) / kChWaves;
+  const int64_t cap = scattered                             ? kWaveRowsScattered
+                      : n >= kWideLevel * (int64_t)nlev ? kWaveRowsWide
+                                                            : kWaveRows;
+  const int64_t srows = std::min<int64_t>(cap, std::max<int64_t>(64, (per + 63) / 64 * 64));
+  P.crows = (int32_t)(kChWaves * srows);
+  P.nchunk = (int32_t)((n + P.crows - 1) / P.crows);
+  const int64_t nwave = (int64_t)P.nchunk * kChWaves;
+  std::vector<int32_t> order(n);
+  {
+    std::vector<int32_t> next(nwave);
+    for (int64_t v = 0; v < nwave; v++) next[v] = (int32_t)std::min<int64_t>(v * srows, n);
+    for (int64_t k = 0; k < n; k++) order[next[at(rows[k]) / srows]++] = rows[k];
   }
-  P.nblk = 0;
-  if (fits && nlev > 0) {
-    blk.push_back(make_int4(nlev, (int32_t)n, (int32_t)nd, 0));
-    P.nblk = (int32_t)blk.size() - 1;
-    P.d_blk = (int4 *)dev_alloc(blk.size() * sizeof(int4));
-    MGX_HIP(hipMemcpy(P.d_blk, blk.data(), blk.size() * sizeof(int4), hipMemcpyHostToDevice));
+  // entries per row and batch: the smallest width that takes 98 % of the rows
+  // in one batch (2, 3 and 13 entries on 5-, 7- and 27-point grids)
+  {
+    const int widths[4] = {2, 4, 8, 14};
+    int64_t over[4] = {0, 0, 0, 0};
+    for (int64_t i = 0; i < n; i++)
+      for (int q = 0; q < 4; q++) over[q] += cnt[i] > widths[q];
+    int q = 0;
+    while (q < 3 && over[q] * 50 > n) q++;
+    P.width = widths[q];
   }
-  if (n > 0) {
-    MGX_HIP(hipMemcpy(L.d_rows, rows.data(), (size_t)n * 4, hipMemcpyHostToDevice));
-    MGX_HIP(hipMemcpy(P.d_rec, rec.data(), (size_t)n * sizeof(int4), hipMemcpyHostToDevice));
+  const uint16_t zero = (uint16_t)slot_zero((uint32_t)P.crows);
+  const int D = P.width;
+  const WidthSizes wd = D == 2   ? width_sizes<2>()
+                        : D == 4 ? width_sizes<4>()
+                        : D == 8 ? width_sizes<8>()
+                                 : width_sizes<14>();
+  const int maxnew = 64 * wd.far;
+  std::vector<int64_t> wave((nwave + 1) * 4);
+  // the waves' batches, by a few threads, each for a run of waves
+  struct Part {
+    std::vector<int4> hdr;
+    std::vector<uint16_t> slot;
+    std::vector<int32_t> dent, ext;
+  };
+  const int nthr = n < 65536 ? 1 : 4;
+  std::vector<Part> part(nthr);
+  auto work = [&](int64_t v0, int64_t v1, Part &out) {
+    std::vector<int4> &hdr = out.hdr;
+    std::vector<uint16_t> &slot = out.slot;
+    std::vector<int32_t> &dent = out.dent, &ext = out.ext;
+    // per row: the wave that last took its value into its ring, and as which
+    std::vector<int32_t> stamp(n, -1);
+    std::vector<int64_t> taken(n);
+    const int64_t mine = std::min<int64_t>(n, (v1 - v0) * srows) + 64;
+    slot.reserve(mine * wd.slots);
+    dent.reserve(mine * D);
+    hdr.reserve(mine / 16);
+    std::vector<int32_t> fresh, ent0(64);
+    for (int64_t v = v0; v < v1; v++) {
+      int64_t *const wv = &wave[v * 4];
+      wv[0] = (int64_t)hdr.size();
+      wv[1] = (int64_t)slot.size() / wd.slots;
+      wv[2] = std::min<int64_t>(v * srows, n);
+      wv[3] = (int64_t)ext.size();
+      const int64_t k1 = std::min<int64_t>(wv[2] + srows, n);
+      const int64_t base = v / kChWaves * P.crows;  // the chunk's first sweep position
+      const uint32_t ring0 = (uint32_t)P.crows + (uint32_t)(v % kChWaves) * kRing;
+      int64_t ntaken = 0;
+      // a value of an earlier chunk: not in the ring, or no longer after the
+      // new ones that may follow (counted from `since`) before it is read?
+      int64_t since = 0;
+      int most = maxnew;
+      auto lacks = [&](int32_t q) {
+        return stamp[q] != (int32_t)v || since + most - taken[q] > kRing;
+      };
+      for (int64_t k = wv[2]; k < k1;) {
+        // the batch's rows: short ones of consecutive levels, or long ones of
+        // one level
+        const bool lng = cnt[order[k]] > D;
+        int64_t ke = k;
+        int longest = 0;
+        uint64_t starts = 0;
+        fresh.clear();
+        since = ntaken;
+        most = lng ? std::max(maxnew, 64 * D) : maxnew;
+        auto take = [&](int32_t q) {
+          stamp[q] = (int32_t)v;
+          taken[q] = ntaken + (int64_t)fresh.size();
+          fresh.push_back(q);
+        };
+        while (ke < k1 && ke - k < 64) {
+          const int32_t i = order[ke];
+          if ((cnt[i] > D) != lng) break;
+          const bool level = ke == k || lev[order[ke - 1]] != lev[i];
+          if (lng && ke > k && (level || longest > 2 * cnt[i] || cnt[i] > 2 * longest)) break;
+          if (!lng) {
+            int news = 0;
+            for_deps(i, [&](int32_t j) { news += at(col[j]) < base && lacks(col[j]); });
+            if (ke > k && (int)fresh.size() + news > maxnew) break;
+            for_deps(i, [&](int32_t j) {
+              if (at(col[j]) < base && lacks(col[j])) take(col[j]);
+            });
+          }
+          if (level) starts |= 1ull << (ke - k);
+          longest = std::max(longest, cnt[i]);
+          ke++;
+        }
+        const int m = (int)(ke - k), parts = std::max(1, (longest + D - 1) / D);
+        for (int l = 0; l < m; l++) ent0[l] = ptr[order[k + l]];
+        for (int pt = 0; pt < parts; pt++) {
+          const size_t s0 = slot.size(), c0 = dent.size();
+          slot.resize(s0 + (size_t)m * wd.slots, zero);
+          dent.resize(c0 + (size_t)m * D, -1);
+          if (lng) {
+            fresh.clear();
+            since = ntaken;
+          }
+          for (int l = 0; l < m; l++) {
+            const int32_t i = order[k + l], left = std::min(cnt[i] - pt * D, D);
+            for (int u = 0; u < left; u++) {
+              int32_t &j = ent0[l];
+              while (!dep_of(filter, i, col[j])) j++;
+              const int32_t q = col[j];
+              dent[c0 + ((size_t)(u / 2) * m + l) * 2 + u % 2] = ent ? (*ent)[j] : j;
+              j++;
+              uint16_t sl;
+              if (at(q) >= base) {
+                sl = (uint16_t)(at(q) - base);
+              } else {
+                if (lng && lacks(q)) {
+                  // (a full batch of new values: one that only takes them)
+                  if ((int)fresh.size() == maxnew) {
+                    push_values(hdr, ext, fresh);
+                    ntaken += maxnew;
+                    fresh.clear();
+                  }
+                  take(q);
+                }
+                sl = (uint16_t)(ring0 + (uint32_t)(taken[q] & (kRing - 1)));
+              }
+              slot[s0 + ((size_t)(u / wd.slot_load) * m + l) * wd.slot_load + u % wd.slot_load] = sl;
+            }
+          }
+          const uint32_t flags = !lng              ? 0u
+                                 : pt == 0         ? (parts == 1 ? kPartFirst | kPartLast : kPartFirst)
+                                 : pt == parts - 1 ? kPartLast
+                                                   : kPartMid;
+          hdr.push_back(make_int4((int32_t)(uint32_t)starts, (int32_t)(uint32_t)(starts >> 32),
+                                  (int32_t)((uint32_t)m | (uint32_t)fresh.size() << 8 | flags), 0));
+          ext.insert(ext.end(), fresh.begin(), fresh.end());
+          ntaken += (int64_t)fresh.size();
+        }
+        k = ke;
+      }
+      while ((int64_t)(hdr.size() - wv[0]) % wd.ahead) hdr.push_back(make_int4(0, 0, 0, 0));
+    }
+  };
+  {
+    std::vector<std::future<void>> run;
+    for (int t = 1; t < nthr; t++)
+      run.push_back(std::async(std::launch::async, work, nwave * t / nthr,
+                               nwave * (t + 1) / nthr, std::ref(part[t])));
+    work(0, nwave / nthr, part[0]);
+    for (auto &r : run) r.get();
   }
-  MGX_HIP(hipMemcpy(L.d_ptr, L.ptr.data(), (size_t)(nlev + 1) * 4, hipMemcpyHostToDevice));
-  MGX_HIP(hipMemcpy(P.d_dcol, dcol.data(), dcol.size() * 4, hipMemcpyHostToDevice));
-  MGX_HIP(hipMemcpy(P.d_dent, dent.data(), dent.size() * 4, hipMemcpyHostToDevice));
+  // behind each other; every array is loaded 64 lanes wide and up to `ahead`
+  // batches past the end
+  Part &last = part.back();
+  wave[nwave * 4] = (int64_t)last.hdr.size();
+  last.hdr.resize(last.hdr.size() + 2 * wd.ahead, make_int4(0, 0, 0, 0));
+  last.slot.resize(last.slot.size() + 64 * wd.slots, zero);
+  last.dent.resize(last.dent.size() + 64 * D, -1);
+  last.ext.resize(last.ext.size() + 64 * (wd.far + 1), 0);
+  int64_t at0[4] = {0, 0, 0, 0};
+  for (int t = 0; t < nthr; t++) {
+    const int64_t v1 = nwave * (t + 1) / nthr + (t + 1 == nthr);  // (and the end of the last)
+    for (int64_t v = nwave * t / nthr; v < v1; v++)
+      for (int q = 0; q < 4; q++) wave[v * 4 + q] += at0[q];
+    at0[0] += (int64_t)part[t].hdr.size();
+    at0[1] += (int64_t)part[t].slot.size() / wd.slots;
+    at0[3] += (int64_t)part[t].ext.size();
+  }
+  std::vector<int32_t> prow(order);
+  prow.resize(n + 128, 0);
+  P.nrow = (int64_t)prow.size();
+  P.ndeps = at0[1] * D;
+  P.d_hdr = upload_parts(part, &Part::hdr);
+  P.d_slot = upload_parts(part, &Part::slot);
+  P.d_dent = upload_parts(part, &Part::dent);
+  P.d_ext = upload_parts(part, &Part::ext);
+  P.d_row = upload(prow);
+  P.d_wave = upload(wave);
   P.built = true;
 }
 
@@ -714,29 +913,28 @@ TriOp tri_prepare(Csr *A, const TriPlan &P, mgx_dtype dt, int fin, const void *v
                   const void *scale, const int32_t *scale_pos) {
   Ctx *c = A->ctx;
   const size_t es = dt == MGX_F64 ? 8 : 4;
-  const int64_t n = A->rows;
   TriOp op;
   op.plan = &P;
   op.fin = fin;
   op.coef = ws_get(c, (size_t)std::max<int64_t>(P.ndeps, 1) * es);
-  op.sc = ws_get(c, (size_t)std::max<int64_t>(n, 1) * es);
-  op.ginit = P.nblk > 0 || P.flow ? ws_get(c, (size_t)std::max<int64_t>(n, 1) * es) : nullptr;
+  op.isc = ws_get(c, (size_t)P.nrow * 2 * es);
   const unsigned gd = (unsigned)((P.ndeps + kBlock - 1) / kBlock);
+  const int64_t n = P.n;
   const unsigned gn = (unsigned)((n + kBlock - 1) / kBlock);
   if (dt == MGX_F64) {
     if (P.ndeps > 0)
       k_tri_pack<double><<<gd, kBlock, 0, c->stream>>>(P.ndeps, P.d_dent, (const double *)vals,
                                                        (double *)op.coef);
     if (n > 0)
-      k_tri_scale<double><<<gn, kBlock, 0, c->stream>>>(n, P.d_rec, (const double *)scale,
-                                                        scale_pos, (double *)op.sc);
+      k_tri_scale<double><<<gn, kBlock, 0, c->stream>>>(n, P.d_row, (const double *)scale,
+                                                        scale_pos, (double *)op.isc);
   } else {
     if (P.ndeps > 0)
       k_tri_pack<float><<<gd, kBlock, 0, c->stream>>>(P.ndeps, P.d_dent, (const float *)vals,
                                                       (float *)op.coef);
     if (n > 0)
-      k_tri_scale<float><<<gn, kBlock, 0, c->stream>>>(n, P.d_rec, (const float *)scale,
-                                                       scale_pos, (float *)op.sc);
+      k_tri_scale<float><<<gn, kBlock, 0, c->stream>>>(n, P.d_row, (const float *)scale,
+                                                       scale_pos, (float *)op.isc);
   }
   MGX_HIP(hipGetLastError());
   return op;
@@ -751,13 +949,13 @@ void tri_run(Csr *A, const TriOp &op, mgx_dtype dt, const void *in, void *out) {
 
 void tri_check_stall(Csr *A) {
   for (TriPlan &P : A->tri) {
-    if (!P.flow || !P.d_ticket) continue;
+    if (!P.d_ticket) continue;
     uint32_t flag = 0;
     MGX_HIP(hipMemcpy(&flag, P.d_ticket + 1, 4, hipMemcpyDeviceToHost));
     if (flag) {
       MGX_HIP(hipMemset(P.d_ticket + 1, 0, 4));
-      set_error("triangular sweep: a row waited more than 2 s for the rows it reads; the "
-                "sweep gave up (result NaN)");
+      set_error("triangular sweep: no row was finished for more than 2 s; the sweep "
+                "gave up (result NaN)");
       throw Error{MGX_ERR_TIMEOUT};
     }
   }
@@ -772,11 +970,14 @@ void levels_free(SorLevels &L) {
 void tri_free(Csr *A) {
   for (TriPlan &P : A->tri) {
     levels_free(P.lev);
+    dev_free(P.d_hdr);
     dev_free(P.d_rec);
     dev_free(P.d_dcol);
+    dev_free(P.d_slot);
     dev_free(P.d_dent);
-    dev_free(P.d_dpos);
-    dev_free(P.d_blk);
+    dev_free(P.d_ext);
+    dev_free(P.d_row);
+    dev_free(P.d_wave);
     dev_free(P.d_ticket);
     P = TriPlan();
   }

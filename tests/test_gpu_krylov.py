@@ -666,6 +666,59 @@ def test_large_wide_level_sweeps_bit_exact(m, ctx, oracle, dtype):
         assert bits_equal(res.rhistory, ref[4])
 
 
+def _banded(n, band, per_row, seed):
+    """n rows of about per_row entries left of the diagonal within `band`
+    columns, and their mirror: rows of 5-8 lower entries, some of them more."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    i = np.repeat(np.arange(n), per_row)
+    j = i - rng.integers(1, band, i.size)
+    L = sp.csr_matrix((rng.uniform(-1, 0, (j >= 0).sum()), (i[j >= 0], j[j >= 0])), shape=(n, n))
+    M = sp.csr_matrix(L + L.T + 4.0 * per_row * sp.eye(n))
+    M.sort_indices()
+    return M.indptr.astype(np.int32), M.indices.astype(np.int32), M.data.copy()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("name", ["grid5", "grid7", "grid7_wide", "banded", "dense_rows",
+                                  "scattered", "scattered_wide"])
+def test_sweeps_across_chunks_bit_exact(m, ctx, oracle, name, dtype):
+    """Triangular sweeps over several chunks of rows, at each width of the
+    batches (2, 4, 8 and 14 entries a row, rows of many more), with long and
+    short row ranges, and with values of earlier chunks by the hundred per
+    batch: ILU(0) apply and two SOR-PCG iterations equal the oracle's serial
+    loops bit for bit."""
+    rp, ci, val = {"grid5": lambda: m.laplacian2d(193, 101),
+                   "grid7": lambda: m.stencil3d(33, 35, 37, 7, 0.1),
+                   "grid7_wide": lambda: m.stencil3d(70, 61, 63, 7, 0.1),
+                   "banded": lambda: _banded(20011, 3000, 7, 1),
+                   "dense_rows": lambda: _banded(9001, 8700, 40, 2),
+                   "scattered": lambda: m.mmatrix(20000),
+                   "scattered_wide": lambda: m.mmatrix(140001)}[name]()
+    val = val.astype(dtype)
+    n = len(rp) - 1
+    b = oracle.random_vector(n, -1.0, 1.0, 91, dtype=dtype)
+    say("chunks", name, dtype.__name__, n)
+    rc, ref = oracle.ilu_precond(rp, ci, val, 5, b)
+    assert rc == 0
+    A = m.CRS(ctx, n, n, rp, ci, val)
+    X = m.Vector(ctx, n=n, dtype=dtype)
+    B = m.Vector(ctx, b, dtype=dtype)
+    assert m.ilu_solve(A, X, B).status == 0
+    assert bits_equal(X.download(), ref)
+    for v in (A, X, B):
+        v.free()
+    oracle.set_sor_omega(1.9)
+    tol = float(1e-30 * oracle.nrm2(b))
+    ref = oracle.solve("cg", rp, ci, val, np.zeros(n, dtype), b, precond=3, tol=tol, maxiter=2,
+                       history=True)
+    res, x = gpu_solve(m, ctx, "cg", rp, ci, val, np.zeros(n, dtype), b, m.PRECOND_SOR, tol,
+                       maxiter=2, mode=m.MODE_REFERENCE, history=2)
+    assert res.status == ref[0] and res.final_iter == ref[2]
+    assert bits_equal(x, ref[1])
+    assert bits_equal(res.rhistory, ref[4])
+
+
 def _wide_then_chain(n_free, n_chain):
     """n_free independent rows (diagonal 4), then a tridiagonal chain
     (4 on the diagonal, -1 beside it): level 0 is wider than a workgroup's
