@@ -10,6 +10,7 @@
 // 512-element tile, whose partial is the block tree of the tile; the blocks
 // then meet in arrive_reduce, which runs stage 2 (lane sums in order, final
 // block tree) spread over the last-arriving blocks.
+#include <cstring>
 #include <mutex>
 
 #include "mgx_device.hpp"
@@ -98,7 +99,10 @@ __global__ __launch_bounds__(kBlock) void k_dot(int64_t n, const T *x, const T *
   const T s = block_tree(p0 + p1, sh);
   if (threadIdx.x == 0) publish_partial(P, tile, s);
   if (arrive_reduce<T, 1, 1>(tick, P, 0, S, ntiles_of(n), tile, tp, sh, res, &flag))
-    if (threadIdx.x == 0) *out = SQ ? (double)sqrt(res[0]) : (double)res[0];
+    if (threadIdx.x == 0)
+      // system scope: out may be host memory that a host thread polls
+      __hip_atomic_store(out, SQ ? (double)sqrt(res[0]) : (double)res[0], __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // m canonical dots <x_r, x_r> of the rows of a row-major block (row r at
@@ -349,14 +353,33 @@ static void *noalloc_scratch(int device) {
   return device >= 0 && device < kNoAllocDevices ? g_scratch_ptr[device] : nullptr;
 }
 
+// The host-returning dot: the kernel's last block stores the result in
+// pinned host memory and this thread watches that word, instead of a copy
+// and a stream synchronisation behind the kernel.  The word holds a
+// signalling NaN until then, which no sum produces.  The watch ends after
+// kWatch: long queues are left to the runtime's wait.
 double dot_host(Ctx *c, mgx_dtype dt, int64_t n, const void *x,
                 const void *y) {
-  double *slot = &c->d_state->rr;
-  launch_dot(c, dt, n, x, y, slot, c->d_tick);
-  MGX_HIP(hipMemcpyAsync(c->h_pinned, slot, sizeof(double),
-                         hipMemcpyDeviceToHost, c->stream));
-  MGX_HIP(hipStreamSynchronize(c->stream));
-  return c->h_pinned[0];
+  if (n <= 0) return 0.0;
+  constexpr uint64_t kUnset = 0x7ff0deadbeef0001ull;
+  constexpr double kWatch = 1e-3;  // seconds
+  double *word = c->h_pinned + kPinnedDot;
+  uint64_t *bits = reinterpret_cast<uint64_t *>(word);
+  __atomic_store_n(bits, kUnset, __ATOMIC_RELEASE);
+  launch_dot(c, dt, n, x, y, word, c->d_tick);
+  uint64_t got = kUnset;
+  const double t0 = seconds_now();
+  for (int spin = 1; (got = __atomic_load_n(bits, __ATOMIC_ACQUIRE)) == kUnset; spin++) {
+    __builtin_ia32_pause();
+    if (spin % 256 == 0 && seconds_now() - t0 > kWatch) {
+      MGX_HIP(hipStreamSynchronize(c->stream));
+      got = __atomic_load_n(bits, __ATOMIC_ACQUIRE);
+      break;
+    }
+  }
+  double v;
+  std::memcpy(&v, &got, sizeof v);
+  return v;
 }
 
 }  // namespace mgx

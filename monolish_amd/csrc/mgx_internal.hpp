@@ -258,6 +258,8 @@ struct Csr {
 };
 constexpr int32_t kEngineSellRow = 256;
 
+constexpr int kPinnedDot = 32;  // on a cache line of its own
+
 struct Ctx {
   int device = 0;
   int32_t batch_iters_per_poll = 0;  // schedule of the last batched solve
@@ -271,7 +273,8 @@ struct Ctx {
   size_t partials_bytes = 0;
   SolveState *d_state = nullptr;     // scratch solve state for BLAS calls
   uint32_t *d_tick = nullptr;        // arrival counters of the BLAS reductions
-  double *h_pinned = nullptr;        // pinned host scalars (64 doubles)
+  double *h_pinned = nullptr;        // pinned host scalars (64 doubles; [0] copies,
+                                     // [kPinnedDot] the dot that the host watches)
   hipEvent_t ev = nullptr;
   // SpMV tuning
   int spmv_rows = 256, spmv_nnz = 2048, spmv_long = 256, xcd_remap = 1;

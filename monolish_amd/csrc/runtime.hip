@@ -205,7 +205,8 @@ int mgx_init(int device, mgx_ctx **out) {
     MGX_HIP(hipMemset(c->d_state, 0, sizeof(SolveState)));
     c->d_tick = (uint32_t *)dev_alloc(kTickWords * sizeof(uint32_t));
     MGX_HIP(hipMemset(c->d_tick, 0, kTickWords * sizeof(uint32_t)));
-    MGX_HIP(hipHostMalloc((void **)&c->h_pinned, 64 * sizeof(double), hipHostMallocDefault));
+    // coherent: the host watches a word of it while a kernel runs (dot_host)
+    MGX_HIP(hipHostMalloc((void **)&c->h_pinned, 64 * sizeof(double), hipHostMallocCoherent));
     MGX_HIP(hipEventCreateWithFlags(&c->ev, hipEventDisableTiming));
     ensure_partials(c, 1 << 20);
     noalloc_scratch_init(device);
