@@ -121,11 +121,16 @@ int mgx_csr_set_plan(mgx_csr *A, int rows_per_block, int nnz_per_block, int xcd_
  * captured hipGraph (re-captured when the set of running systems changes);
  * 0 (default): direct kernel launches */
 int mgx_set_graphs(mgx_ctx *ctx, int enable);
-/* 1: a fused CG solve of one system small enough for the two-kernel
- * iteration runs its iterations inside one cooperative launch (grid barriers
- * between the stages); 0 (default, measured faster on MI355X): one launch per
- * stage; a value above 1 enables it with at most that many blocks (each
- * block then owns several 128-row quarters) */
+/* How single fused solves (one CG or BiCGSTAB system, no triangular
+ * preconditioner) run.  Until this is called: systems of at most 7 entries a
+ * row and 524287 rows (BiCGSTAB: 262144) run whole in one cooperative launch,
+ * held in registers; others one launch per stage.  0: always one launch per stage.
+ * 1: as before the call, and other CG systems small enough for the
+ * two-kernel iteration also run in one cooperative launch (grid barriers
+ * between the stages).  A value above 1: CG systems small enough for the
+ * two-kernel iteration, in one cooperative launch of at most that many
+ * blocks (each then owns several 128-row quarters).  The results are the
+ * same bits in every form. */
 int mgx_set_persistent(mgx_ctx *ctx, int enable);
 
 /* ---- vectors: vector<T>::send/recv/nonfree_recv/device_free ------------- */

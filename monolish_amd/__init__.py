@@ -712,8 +712,9 @@ def set_graphs(ctx: Context, enable: bool):
 
 
 def set_persistent(ctx: Context, enable, max_blocks: int = 0):
-    """Run single small fused CG solves in one cooperative launch (default off);
-    max_blocks > 1 caps its grid."""
+    """Run single small fused solves in one cooperative launch (False: one
+    launch per stage; never called: where the system fits the registers);
+    max_blocks > 1 caps a CG solve's grid."""
     check(_lib.mgx_set_persistent(ctx.handle, int(max_blocks) if enable and max_blocks > 1
                                   else int(bool(enable))))
 

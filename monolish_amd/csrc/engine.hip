@@ -131,6 +131,7 @@ template <class T> Engine<T>::~Engine() {
   dev_free(d_tiles_[0]);
   dev_free(d_tiles_[1]);
   dev_free(d_gs_);
+  dev_free(d_res_);
   dev_free(d_ticks_);
   dev_free(d_stage_);
   dev_free(d_ptiles_);
@@ -245,7 +246,9 @@ int Engine<T>::add(Csr *A, const void *val, T *x, const T *b, const SolveCfg &cf
     d.sci = sl->d_sci;
     d.sval = static_cast<const T *>(sl->d_val);
   }
-  d.lf = cfg.method == kMethodCG && !d.split && nt <= kRedGroups && !c_->use_persistent ? 1 : 0;
+  d.lf = cfg.method == kMethodCG && !d.split && nt <= kRedGroups && c_->use_persistent <= 0
+             ? 1
+             : 0;
   d.vec = ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
   d.method = cfg.method;
   d.tol_scale = cfg.tol_relative ? cfg.tol : 0.0;
@@ -464,7 +467,7 @@ template <class T> void Engine<T>::step(int iters) {
 }
 
 template <class T> bool Engine<T>::persistent_ok(int slot) const {
-  if (!c_->use_persistent || active_.size() != 1 || active_[0] != slot) return false;
+  if (c_->use_persistent <= 0 || active_.size() != 1 || active_[0] != slot) return false;
   const SysDesc<T> &d = h_sys_[slot];
   return method_[slot] == kMethodCG && !d.split && !d.once && !d.lf;
 }
@@ -492,6 +495,46 @@ template <class T> void Engine<T>::run_persistent(int slot) {
     std::memcpy(&err, c_->h_pinned, sizeof err);
     MGX_REQUIRE(err == 0, "persistent CG: a grid barrier wait timed out");
     if (!poll().empty()) return;
+  }
+}
+
+// A lone system of short rows runs resident unless the caller asked for
+// launch-per-stage solves, for a capped grid or for graph replay.  Measured on
+// one system, FP64, resident against the launches: see resident.hip.
+template <class T> bool Engine<T>::resident_ok(int slot) const {
+  if (c_->use_persistent == 0 || c_->use_persistent > 1 || c_->use_graphs) return false;
+  if (active_.size() != 1 || active_[0] != slot) return false;
+  return !h_sys_[slot].split && resident_fits(c_, csr_[slot], method_[slot]);
+}
+
+template <class T> bool Engine<T>::run_resident(int slot) {
+  MGX_REQUIRE(resident_ok(slot), "engine: not a resident solve");
+  flush_pending();
+  const int64_t nt = h_sys_[slot].ntiles;
+  const size_t bytes = resident_bytes(nt);
+  if (bytes > res_cap_) {
+    dev_free(d_res_);
+    d_res_ = nullptr;
+    d_res_ = dev_alloc(bytes);
+    res_cap_ = bytes;
+  }
+  // a launch ends after this many iterations (a second or two); the host
+  // looks at the state and launches again if the solve is still running
+  constexpr int64_t kPerLaunch = 1 << 17;
+  for (bool fresh = true;; fresh = false) {
+    resident_launch<T>(c_, method_[slot], d_sys_ + slot, nt, csr_[slot]->plan.max_row, d_res_,
+                       d_stopped_, kPerLaunch);
+    uint32_t err = 0;
+    MGX_HIP(hipMemcpyAsync(c_->h_pinned + 1, d_res_, sizeof(uint32_t), hipMemcpyDeviceToHost,
+                           c_->stream));
+    const bool stopped = !poll().empty();
+    std::memcpy(&err, c_->h_pinned + 1, sizeof err);
+    if (err != 0) {
+      if (fresh) return false;
+      set_error("resident solve: the blocks of a launch did not meet within 2 s");
+      throw Error{MGX_ERR_TIMEOUT};
+    }
+    if (stopped) return true;
   }
 }
 

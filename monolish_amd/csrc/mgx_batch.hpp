@@ -121,6 +121,18 @@ template <class T>
 void batch_launch_cg_persist(Ctx *c, const SysDesc<T> *sys, GridSync *gs, int grid,
                              int32_t *stopped, int lds_entries, int max_iters);
 
+// resident solves (resident.hip): the system's rows fit the registers of one
+// cooperative launch (rows of at most 7 entries; CG at most 1024 tiles,
+// BiCGSTAB at most 512)
+bool resident_fits(const Ctx *c, const Csr *A, int method);
+size_t resident_bytes(int64_t ntiles);  // scratch of a launch
+// up to max_iters iterations of the single system sys[0] (CG or BiCGSTAB);
+// the first word of scratch is nonzero afterwards when a wait gave up: x
+// and the solve state are then as they were
+template <class T>
+void resident_launch(Ctx *c, int method, const SysDesc<T> *sys, int64_t ntiles, int max_row,
+                     void *scratch, int32_t *stopped, int64_t max_iters);
+
 // set-up of newly admitted systems: scatter their staged descriptors and
 // states into their slots, then (over the list of their tiles) M = 1/diag,
 // r = b - A x with z = M r or r0 = r, the relative tolerances, <z,r> or
@@ -231,6 +243,11 @@ template <class T> class Engine {
   bool persistent_ok(int slot) const;
   // iterate that system to its end with the persistent kernel
   void run_persistent(int slot);
+  // the one running system fits a resident solve and the context allows it
+  bool resident_ok(int slot) const;
+  // iterate it to its end that way; false when the blocks did not meet in
+  // time (x untouched, the work vectors not)
+  bool run_resident(int slot);
 
  private:
   void rebuild_lists();
@@ -264,6 +281,8 @@ template <class T> class Engine {
   int host_running_ = 0;
   int lds_entries_ = 0;
   GridSync *d_gs_ = nullptr;      // grid barrier of the persistent kernel
+  void *d_res_ = nullptr;         // scratch of the resident solves
+  size_t res_cap_ = 0;
   uint32_t *d_ticks_ = nullptr;   // kTickWords arrival counters per slot
   std::vector<int> pending_;      // slots added since the last launch
   std::vector<char> rel_;         // per slot: relative tolerance

@@ -17,12 +17,37 @@
 
 namespace mgx {
 
-template <class T> __device__ __forceinline__ T wave_tree(T v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    T o = __shfl_down(v, off, 64);
-    v = v + o;
+// v of another lane, by the register-to-register moves (no LDS round trip):
+// lanes below 32 / 16 get lane l + OFF for OFF = 32 / 16 (swaps of half waves
+// and rows), lanes of a row of 16 get lane l + OFF of that row below; other
+// lanes get something else
+template <int OFF> __device__ __forceinline__ uint32_t lane_up(uint32_t v) {
+  if constexpr (OFF == 32)
+    return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+  else if constexpr (OFF == 16)
+    return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+  else
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x100 + OFF, 0xf, 0xf, true);
+}
+template <int OFF, class T> __device__ __forceinline__ T lane_up_t(T v) {
+  if constexpr (sizeof(T) == 8) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint64_t r = (uint64_t)lane_up<OFF>((uint32_t)(b >> 32)) << 32 |
+                       lane_up<OFF>((uint32_t)b);
+    return __builtin_bit_cast(T, r);
+  } else {
+    return __builtin_bit_cast(T, lane_up<OFF>(__builtin_bit_cast(uint32_t, v)));
   }
+}
+
+// the wave's sum in lane 0 (other lanes: unspecified)
+template <class T> __device__ __forceinline__ T wave_tree(T v) {
+  v = v + lane_up_t<32>(v);
+  v = v + lane_up_t<16>(v);
+  v = v + lane_up_t<8>(v);
+  v = v + lane_up_t<4>(v);
+  v = v + lane_up_t<2>(v);
+  v = v + lane_up_t<1>(v);
   return v;
 }
 

@@ -279,8 +279,10 @@ struct Ctx {
   // SpMV tuning
   int spmv_rows = 256, spmv_nnz = 2048, spmv_long = 256, xcd_remap = 1;
   int use_graphs = 0;  // replay fused iterations from a captured hipGraph
-  int use_persistent = 0;  // single small CG solves in one cooperative launch
-                           // (> 1: also the largest grid it may use)
+  // single small solves in one cooperative launch: -1 the library's choice
+  // (resident solves where they fit), 0 never, 1 wherever a form fits, > 1
+  // CG only, on at most that many blocks
+  int use_persistent = -1;
   // fused-engine state owned by the context (engine.hip)
   void *pool = nullptr;   // DevicePool for solver work vectors
   void *eng64 = nullptr;  // Engine<double> for single fused solves

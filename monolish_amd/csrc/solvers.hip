@@ -271,9 +271,17 @@ SolveOut fused_solve(int method, Csr *A, const void *val, T *x, const T *b, int 
   cfg.maxiter = maxiter;
   cfg.rhist = rh;
   cfg.rhist_len = rlen;
-  const int slot = eng.add(A, val, x, b, cfg);
+  int slot = eng.add(A, val, x, b, cfg);
   MGX_REQUIRE(slot >= 0, "fused solve: out of device memory for the work vectors");
-  if (eng.persistent_ok(slot)) {
+  bool done = false;
+  if (eng.resident_ok(slot) && !(done = eng.run_resident(slot))) {
+    // set the system up again for the launches
+    eng.release(slot);
+    slot = eng.add(A, val, x, b, cfg);
+    MGX_REQUIRE(slot >= 0, "fused solve: out of device memory for the work vectors");
+  }
+  if (done) {
+  } else if (eng.persistent_ok(slot)) {
     eng.run_persistent(slot);
   } else {
     const int every = check_every > 0 ? check_every : 32;

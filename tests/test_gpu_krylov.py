@@ -239,6 +239,58 @@ def test_cg_persistent_kernel(m, ctx, oracle, blocks):
         m.set_persistent(ctx, False)
 
 
+def _ring(n, reach, seed):
+    """n rows of 2 reach + 1 entries (fewer when n is small): a ring with
+    neighbours up to `reach` away, unsymmetric values, diagonal 3 reach."""
+    rng = np.random.default_rng(seed)
+    off = np.arange(-reach, reach + 1)
+    rows = [np.unique((i + off) % n) for i in range(min(n, 4 * reach + 4))]
+    if n > 4 * reach + 4:
+        cols = np.sort((np.arange(n)[:, None] + off[None, :]) % n, axis=1)
+        rp = np.arange(0, n * off.size + 1, off.size, dtype=np.int32)
+        ci = cols.reshape(-1).astype(np.int32)
+    else:
+        rp = np.zeros(n + 1, np.int32)
+        rp[1:] = np.cumsum([len(r) for r in rows])
+        ci = np.concatenate(rows).astype(np.int32)
+    val = rng.uniform(-1, 0, ci.size)
+    row = np.repeat(np.arange(n), np.diff(rp))
+    val[ci == row] = 3.0 * reach
+    return rp, ci, val
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,reach", [(1, 2), (2, 2), (511, 2), (513, 3), (1537, 1), (131072, 2),
+                                     (131073, 3), (262145, 2), (262145, 3), (524287, 2)])
+def test_resident_solves_equal_launches(m, oracle, n, reach, dtype):
+    """One system in one cooperative launch, at the edges of its shapes (one
+    tile, tiles side by side, two rounds, the largest size), rows of up to 5
+    and 7 entries, with and without Jacobi: x, status, residual and history
+    equal the launch-per-stage form's bit for bit, and the oracle's for the
+    smaller ones."""
+    rp, ci, val = _ring(n, reach, n)
+    val = val.astype(dtype)
+    b = oracle.random_vector(n, -1.0, 1.0, 5, dtype=dtype)
+    say("resident", n, reach, dtype.__name__)
+    tol = float((1e-9 if dtype == np.float64 else 1e-4) * oracle.nrm2(b))
+    with m.Context(0) as own, m.Context(0) as staged:
+        m.set_persistent(staged, False)
+        for method in ("cg", "bicgstab"):
+            for prec, iters in ((m.PRECOND_JACOBI, 60), (m.PRECOND_NONE, 3)):
+                out = [gpu_solve(m, c, method, rp, ci, val, np.zeros(n, dtype), b, prec, tol,
+                                 maxiter=iters, mode=m.MODE_FUSED, history=iters)
+                       for c in (own, staged)]
+                (r1, x1), (r2, x2) = out
+                assert (r1.status, r1.final_iter) == (r2.status, r2.final_iter)
+                assert bits_equal(x1, x2) and bits_equal(r1.rhistory, r2.rhistory)
+                assert r1.final_resid == r2.final_resid or r1.final_resid != r1.final_resid
+                if n < 2000:
+                    ref = oracle.solve(method, rp, ci, val, np.zeros(n, dtype), b, precond=prec,
+                                       tol=tol, maxiter=iters, history=True)
+                    assert r1.status == ref[0] and r1.final_iter == ref[2]
+                    assert bits_equal(x1, ref[1])
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_cg_fused_large_split_iteration(m, ctx, oracle, dtype):
     """n >= 2^19 rows: the fused solver runs the split iteration (p update,
