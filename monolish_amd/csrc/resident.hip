@@ -23,15 +23,15 @@
 // of step k + 2 comes after the clearing has completed).  The vector that the
 // next SpMV gathers is stored before the partials are published, so the
 // same step makes it visible.  Each partial is published once per XCD, so
-// that an XCD's blocks poll lines of their own (one copy for all: 10.6 us an
-// iteration on 256^2 instead of 8.1).  Arithmetic and order are those of the
+// that an XCD's blocks poll lines of their own (one copy for all: 2.5 us more
+// an iteration on 256^2).  Arithmetic and order are those of the
 // launch-per-stage kernels (batch.hip), so the bits are the same.
 //
-// Per iteration, FP64, resident / launches (us): CG, 5-point 20^2 5.9 / 14.9,
-// 256^2 6.7 / 13.5, 500^2 9.9 / 33.9, 700^2 15.2 / 49.0; 7-point 30^3 7.5 /
-// 15.4, 60^3 10.4 / 36.5, 80^3 21.4 / 56.9 (two rounds of tiles, some
-// registers spilled); BiCGSTAB, 5-point 100^2 9.7 / 28.7, 500^2 16.0 / 56.3;
-// 7-point 60^3 18.0 / 53.9.  What is left of an iteration is latency: a store
+// Per iteration, FP64, resident / launches (us): CG, 5-point 20^2 4.5 / 14.5,
+// 256^2 4.9 / 13.4, 500^2 7.8 / 34.6, 700^2 11.8 / 49.3; 7-point 30^3 5.5 /
+// 15.3, 60^3 8.5 / 36.1, 80^3 19.5 / 57.4 (two rounds of tiles, some
+// registers spilled); BiCGSTAB, 5-point 100^2 8.1 / 28.3, 500^2 13.9 / 56.3;
+// 7-point 60^3 17.1 / 53.5.  What is left of an iteration is latency: a store
 // to memory, a poll, a gather, per step about 2 us.
 #include <algorithm>
 
@@ -75,11 +75,30 @@ __global__ __launch_bounds__(kBlock) void k_res_clear(typename Slot<T>::U *slots
   if (i == 0) *err = 0u;
 }
 
+// the descriptor's fields, read once by scalar loads into registers (read
+// through a reference they were loaded anew, with a wait for everything in
+// flight, at each use: 1.5 to 3.5 us more per iteration)
+template <class T> struct ResDesc {
+  const int32_t *rp, *ci;
+  const T *val, *M;
+  T *x, *r, *z, *pa, *pb, *r0, *va;
+  double *rhist;
+  int64_t rhist_len, n, ntiles;
+  SolveState *st;
+  __device__ __forceinline__ explicit ResDesc(const SysDesc<T> *sys) {
+    typedef const __attribute__((address_space(4))) SysDesc<T> C;
+    C *c = (C *)sys;
+    rp = c->rp, ci = c->ci, val = c->val, M = c->M, x = c->x, r = c->r, z = c->z, pa = c->pa;
+    pb = c->pb, r0 = c->r0, va = c->va, rhist = c->rhist, rhist_len = c->rhist_len;
+    n = c->n, ntiles = c->ntiles, st = c->st;
+  }
+};
+
 // TT tiles side by side in a block (256 threads each), TR rounds of them; KE:
 // entries a row holds at most
 template <class T, int TT, int TR, int KE> struct Resident {
   using U = typename Slot<T>::U;
-  const SysDesc<T> &d;
+  const ResDesc<T> &d;
   U *slots;       // 3 sets x kCopies x 2 sums x ntiles
   uint32_t *err;  // raised when a wait gave up
   T *sh;          // LDS: TT * TR * 8 wave sums, then 8, then 2 results
@@ -91,7 +110,7 @@ template <class T, int TT, int TR, int KE> struct Resident {
   int len[TR][2];
   uint32_t step = 0;
 
-  __device__ __forceinline__ Resident(const SysDesc<T> &desc, U *s, uint32_t *e, T *lds, int *b)
+  __device__ __forceinline__ Resident(const ResDesc<T> &desc, U *s, uint32_t *e, T *lds, int *b)
       : d(desc), slots(s), err(e), sh(lds), bad(b) {
     const int t = threadIdx.x & (kBlock - 1), g = threadIdx.x / kBlock;
 #pragma unroll
@@ -271,7 +290,7 @@ __global__ __launch_bounds__(kBlock *TT) void k_resident_cg(const SysDesc<T> *sy
                                                             int64_t max_iters) {
   __shared__ T sh[8 * TT * TR + 8];
   __shared__ int bad;
-  const SysDesc<T> &d = sys[0];
+  const ResDesc<T> d(sys);
   SolveState *st = d.st;
   if (st->status != kStatRunning) return;
   if (threadIdx.x == 0) bad = 0;
@@ -395,7 +414,7 @@ __global__ __launch_bounds__(kBlock *TT) void k_resident_bcg(const SysDesc<T> *s
                                                              int64_t max_iters) {
   __shared__ T sh[8 * TT * TR + 8];
   __shared__ int bad;
-  const SysDesc<T> &d = sys[0];
+  const ResDesc<T> d(sys);
   SolveState *st = d.st;
   if (st->status != kStatRunning) return;
   if (threadIdx.x == 0) bad = 0;
