@@ -299,9 +299,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(const SysDesc<T> *sys,
   const int64_t R0 = d.row0 + qi * kQuarter;
   const int64_t R1 = min(d.row0 + d.n, R0 + kQuarter);
   if (d.sell)
-    tile_sell(d, R0, R1, qloc, d.q, pv);
+    tile_sell<T>(d, R0, R1, qloc, d.q, pv);
   else
-    tile_spmv(d, qi, R0, prod, qloc, d.q, sh, pv);
+    tile_spmv<T>(d, qi, R0, prod, qloc, d.q, sh, pv);
   const int t = threadIdx.x;
   T acc0 = 0, acc1 = 0;
   if (t < 64) {
@@ -320,10 +320,10 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv(const SysDesc<T> *sys,
   T s = wave_tree(acc0 + acc1);
   if (d.lf) {
     // k_cg_update finishes <p, q>
-    if (t == 0) publish_partial(d.P, lf_pq_off(d) + qi, s);
+    if (t == 0) publish_partial<T>(d.P, lf_pq_off(d) + qi, s);
     return;
   }
-  if (t == 0) publish_partial(d.P, qi, s);
+  if (t == 0) publish_partial<T>(d.P, qi, s);
   if (arrive_reduce<T, 1, 4>(d.tick, d.P, 0, d.S, d.ntiles, qi, prod, sh, res, &flag)) {
     if (t == 0) {
       const T pq = res[0];
@@ -429,8 +429,8 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(const SysDesc<T> *sys,
   T rr_a = rr2[0] + rr2[1];
   block_tree2(zr_a, rr_a, sh);
   if (t == 0) {
-    publish_partial(d.P, tile, zr_a);
-    publish_partial(d.P, d.ntiles + tile, rr_a);
+    publish_partial<T>(d.P, tile, zr_a);
+    publish_partial<T>(d.P, d.ntiles + tile, rr_a);
   }
   if (d.lf) {
     // the next iteration's opening kernel finishes <z,r> and <r,r>
@@ -461,7 +461,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_finish(const SysDesc<T> *sys,
   if (d.acc64) {
     // FP64 partials and scalars (mixed-precision inner CG)
     __shared__ double shd[8];
-    const double *Pd = reinterpret_cast<const double *>(d.P);
+    const double *Pd = reinterpret_cast<const double *>(static_cast<T *>(d.P));
     if (stage == 0) {
       const double pq = reduce_partials(Pd, d.ntiles, shd);
       if (threadIdx.x == 0) {
@@ -477,16 +477,16 @@ __global__ __launch_bounds__(kBlock) void k_cg_finish(const SysDesc<T> *sys,
     return;
   }
   if (stage == 0) {
-    const T pq = reduce_partials(d.P, d.ntiles, sh);
+    const T pq = reduce_partials<T>(d.P, d.ntiles, sh);
     if (threadIdx.x == 0) {
       const T zr = (T)st->zr;
       st->pq = (double)pq;
       st->alpha = (double)(zr / pq);
     }
   } else {
-    const T zr_new = reduce_partials(d.P, d.ntiles, sh);
+    const T zr_new = reduce_partials<T>(d.P, d.ntiles, sh);
     __syncthreads();
-    const T rr = reduce_partials(d.P + d.ntiles, d.ntiles, sh);
+    const T rr = reduce_partials<T>(d.P + d.ntiles, d.ntiles, sh);
     if (threadIdx.x == 0) cg_finish<T>(d, st, zr_new, rr, stopped);
   }
 }
@@ -586,7 +586,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_persist(const SysDesc<T> *sys, Gr
     for (int64_t qi = blk; qi < nq; qi += G) {
       const int64_t R0 = qi * kQuarter;
       const int64_t R1 = min(d.n, R0 + kQuarter);
-      tile_spmv(d, qi, R0, prod, qloc, d.q, sh, pv);
+      tile_spmv<T>(d, qi, R0, prod, qloc, d.q, sh, pv);
       T acc0 = 0, acc1 = 0;
       if (t < 64) {
         const int64_t i0 = R0 + 2 * t;
@@ -602,11 +602,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_persist(const SysDesc<T> *sys, Gr
         }
       }
       const T s = wave_tree(acc0 + acc1);
-      if (t == 0) publish_partial(d.P, qi, s);
+      if (t == 0) publish_partial<T>(d.P, qi, s);
       __syncthreads();  // qloc and prod are reused by the next quarter
     }
     if (grid_arrive(gs, G, ngroups, blk, ++gen, &flag)) {
-      const T pq = reduce_quarters(d.P, d.ntiles, sh);
+      const T pq = reduce_quarters<T>(d.P, d.ntiles, sh);
       if (t == 0) {
         const T zr = (T)sld(&st->zr);
         sst(&st->pq, (double)pq);
@@ -645,14 +645,14 @@ __global__ __launch_bounds__(kBlock) void k_cg_persist(const SysDesc<T> *sys, Gr
       const T zr_w = wave_tree(zr2[0] + zr2[1]);
       const T rr_w = wave_tree(rr2[0] + rr2[1]);
       if (t == 0) {
-        publish_partial(d.P, qi, zr_w);
-        publish_partial(d.P, nq + qi, rr_w);
+        publish_partial<T>(d.P, qi, zr_w);
+        publish_partial<T>(d.P, nq + qi, rr_w);
       }
     }
     if (grid_arrive(gs, G, ngroups, blk, ++gen, &flag)) {
-      const T zr_new = reduce_quarters(d.P, d.ntiles, sh);
+      const T zr_new = reduce_quarters<T>(d.P, d.ntiles, sh);
       __syncthreads();
-      const T rr = reduce_quarters(d.P + nq, d.ntiles, sh);
+      const T rr = reduce_quarters<T>(d.P + nq, d.ntiles, sh);
       if (t == 0) cg_finish<T>(d, st, zr_new, rr, stopped);
       grid_release(gs, gen);
     } else if (!grid_wait(gs, gen, &flag)) {
@@ -787,7 +787,7 @@ __device__ __forceinline__ void split_publish(const SysDesc<T> &d, const R (*lan
   const int64_t tile = (int64_t)blockIdx.x * kSplitTiles + threadIdx.x;
   if ((int)threadIdx.x < kSplitTiles && tile < d.ntiles) {
     const R *w = sh + threadIdx.x * 8;
-    R *P = reinterpret_cast<R *>(d.P);
+    R *P = reinterpret_cast<R *>(static_cast<T *>(d.P));
 #pragma unroll
     for (int r = 0; r < NR; r++) {
       const R lo = w[4 * r] + w[4 * r + 1], hi = w[4 * r + 2] + w[4 * r + 3];
@@ -943,9 +943,9 @@ __global__ __launch_bounds__(kBlock) void k_bcg_spmv1(const SysDesc<T> *sys,
   const int64_t R0 = d.row0 + qi * kQuarter;
   const int64_t R1 = min(d.row0 + d.n, R0 + kQuarter);
   if (d.sell)
-    tile_sell(d, R0, R1, qloc, v_new, phv);
+    tile_sell<T>(d, R0, R1, qloc, v_new, phv);
   else
-    tile_spmv(d, qi, R0, prod, qloc, v_new, sh, phv);
+    tile_spmv<T>(d, qi, R0, prod, qloc, v_new, sh, phv);
   const int t = threadIdx.x;
   T acc[2] = {0, 0};
   if (t < 64) {
@@ -964,7 +964,7 @@ __global__ __launch_bounds__(kBlock) void k_bcg_spmv1(const SysDesc<T> *sys,
     }
   }
   T s = wave_tree(acc[0] + acc[1]);
-  if (t == 0) publish_partial(d.P, qi, s);
+  if (t == 0) publish_partial<T>(d.P, qi, s);
   if (arrive_reduce<T, 1, 4>(d.tick, d.P, 0, d.S, d.ntiles, qi, prod, sh, res, &flag)) {
     if (t == 0) {
       const T vr0 = res[0];
@@ -1013,9 +1013,9 @@ __global__ __launch_bounds__(kBlock) void k_bcg_spmv2(const SysDesc<T> *sys,
   const int64_t R0 = d.row0 + qi * kQuarter;
   const int64_t R1 = min(d.row0 + d.n, R0 + kQuarter);
   if (d.sell)
-    tile_sell(d, R0, R1, qloc, d.t, shv);
+    tile_sell<T>(d, R0, R1, qloc, d.t, shv);
   else
-    tile_spmv(d, qi, R0, prod, qloc, d.t, sh, shv);
+    tile_spmv<T>(d, qi, R0, prod, qloc, d.t, sh, shv);
   const int t = threadIdx.x;
   T ts2[2] = {0, 0}, tt2[2] = {0, 0};
   if (t < 64) {
@@ -1041,8 +1041,8 @@ __global__ __launch_bounds__(kBlock) void k_bcg_spmv2(const SysDesc<T> *sys,
   T ts_a = wave_tree(ts2[0] + ts2[1]);
   T tt_a = wave_tree(tt2[0] + tt2[1]);
   if (t == 0) {
-    publish_partial(d.P, qi, ts_a);
-    publish_partial(d.P, 4 * d.ntiles + qi, tt_a);
+    publish_partial<T>(d.P, qi, ts_a);
+    publish_partial<T>(d.P, 4 * d.ntiles + qi, tt_a);
   }
   if (arrive_reduce<T, 2, 4>(d.tick, d.P, 4 * d.ntiles, d.S, d.ntiles, qi, prod, sh, res,
                              &flag)) {
@@ -1188,8 +1188,8 @@ __global__ __launch_bounds__(kBlock) void k_bcg_update(const SysDesc<T> *sys,
   T rq_a = rq2[0] + rq2[1];
   block_tree2(rr_a, rq_a, sh);
   if (t == 0) {
-    publish_partial(d.P, tile, rr_a);
-    publish_partial(d.P, d.ntiles + tile, rq_a);
+    publish_partial<T>(d.P, tile, rr_a);
+    publish_partial<T>(d.P, d.ntiles + tile, rq_a);
   }
   if (arrive_reduce<T, 2, 1>(d.tick, d.P, d.ntiles, d.S, d.ntiles, tile, tp, sh, res,
                              &flag)) {
@@ -1256,7 +1256,7 @@ __global__ __launch_bounds__(kBlock) void k_setup_diag(const SysDesc<T> *sys,
   int64_t tile;
   const SysDesc<T> &d = locate(sys, tiles, b, tile);
   if (!d.M) return;
-  T *M = const_cast<T *>(d.M);
+  T *M = const_cast<T *>(static_cast<const T *>(d.M));
   const int t = threadIdx.x;
   for (int half = 0; half < 2; half++) {
     const int64_t r0 = tile * kTile + half * kBlock;
@@ -1305,7 +1305,7 @@ __global__ __launch_bounds__(kBlock) void k_setup_r(const SysDesc<T> *sys, const
   const int64_t R1 = min(d.n, R0 + kQuarter);
   const T *x = d.x;
   T *scratch = d.method == kMethodCG ? d.q : d.t;
-  tile_spmv(d, qi, R0, prod, qloc, scratch, sh, [&](int64_t c) { return x[c]; });
+  tile_spmv<T>(d, qi, R0, prod, qloc, scratch, sh, [&](int64_t c) { return x[c]; });
   const int64_t i = R0 + threadIdx.x;
   if (threadIdx.x < kQuarter && i < R1) {
     const T rv = d.b[i] - qloc[threadIdx.x];
@@ -1352,7 +1352,7 @@ __global__ __launch_bounds__(kBlock) void k_sys_dot(const SysDesc<T> *sys,
     if (i0 + 1 < R1) p1 = xv[i0 + 1] * yv[i0 + 1];
   }
   T s = block_tree(p0 + p1, sh);
-  if (threadIdx.x == 0) publish_partial(d.P, tile, s);
+  if (threadIdx.x == 0) publish_partial<T>(d.P, tile, s);
   if (arrive_reduce<T, 1, 1>(d.tick, d.P, 0, d.S, d.ntiles, tile, tp, sh, res, &flag)) {
     if (threadIdx.x == 0) {
       const T v = res[0];

@@ -172,7 +172,7 @@ int Engine<T>::add(Csr *A, const void *val, T *x, const T *b, const SolveCfg &cf
   SysDesc<T> d;
   std::memset(&d, 0, sizeof d);
   bool ok = true;
-  auto need = [&](T *&dst) {
+  auto need = [&](GPtr<T> &dst) {
     dst = take(vb);
     ok = ok && dst != nullptr;
   };
@@ -180,9 +180,9 @@ int Engine<T>::add(Csr *A, const void *val, T *x, const T *b, const SolveCfg &cf
   need(d.pa);
   need(d.pb);
   if (cfg.precond == MGX_PRECOND_JACOBI) {
-    T *m = nullptr;
+    GPtr<T> m = nullptr;
     need(m);
-    d.M = m;
+    d.M = (T *)m;
   }
   if (cfg.method == kMethodCG) {
     need(d.z);
@@ -385,7 +385,7 @@ template <class T> void Engine<T>::launch_iters(int iters) {
           // fused SpMV forms the <p, q> partials
           MGX_REQUIRE(spmv_sell_pq(csr_[s], val_[s], DTof<T>::v, h.pa, h.q, h.P,
                                    &d_states_[s].status, h.acc64 != 0,
-                                   reinterpret_cast<const float *>(h.dcorr)),
+                                   reinterpret_cast<const float *>(static_cast<const T *>(h.dcorr))),
                       "solver: the matrix's SpMV plan changed during a solve");
         } else {
           launch_spmv(csr_[s], val_[s], DTof<T>::v, h.pa, h.q, 1.0, 0.0, false,

@@ -88,9 +88,20 @@ template <class T> struct ResDesc {
   __device__ __forceinline__ explicit ResDesc(const SysDesc<T> *sys) {
     typedef const __attribute__((address_space(4))) SysDesc<T> C;
     C *c = (C *)sys;
-    rp = c->rp, ci = c->ci, val = c->val, M = c->M, x = c->x, r = c->r, z = c->z, pa = c->pa;
-    pb = c->pb, r0 = c->r0, va = c->va, rhist = c->rhist, rhist_len = c->rhist_len;
-    n = c->n, ntiles = c->ntiles, st = c->st;
+    rp = (decltype(rp))c->rp.p;
+    ci = (decltype(ci))c->ci.p;
+    val = (decltype(val))c->val.p;
+    M = (decltype(M))c->M.p;
+    x = (decltype(x))c->x.p;
+    r = (decltype(r))c->r.p;
+    z = (decltype(z))c->z.p;
+    pa = (decltype(pa))c->pa.p;
+    pb = (decltype(pb))c->pb.p;
+    r0 = (decltype(r0))c->r0.p;
+    va = (decltype(va))c->va.p;
+    rhist = (decltype(rhist))c->rhist.p;
+    st = (SolveState *)c->st.p;
+    rhist_len = c->rhist_len, n = c->n, ntiles = c->ntiles;
   }
 };
 
