@@ -198,6 +198,11 @@ struct SpmvPlan {
     // row lengths, min(len, 255): the kernels read row_ptr only for rows
     // of 255 entries or more
     uint8_t *d_len = nullptr;
+    // row patterns (mgx_sell.hpp), where the matrix has few enough: a byte
+    // per row and the table (npat 0: none)
+    uint8_t *d_pat = nullptr;
+    int32_t *d_ptab = nullptr;
+    int32_t npat = 0, pstride = 0;
   };
   int32_t sell = 0;
   Sliced sl, sl32;

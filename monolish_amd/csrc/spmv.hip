@@ -235,6 +235,107 @@ __global__ void k_sell_fill(int64_t rows, const int32_t *__restrict__ rp,
   }
 }
 
+// the slice of row r, the same in a wave's lanes (blocks hold whole slices)
+__device__ __forceinline__ int64_t wave_slice(int64_t r) {
+  return __builtin_amdgcn_readfirstlane((int32_t)(r / kSlice));
+}
+
+// Finding the row patterns: rows enter a 64-bit hash of their differences
+// into a small open table (k_pat_find; a row that finds more than cap of them
+// raises `fail`, and the rows after it return at once), the table's entries
+// get their ids and their row of the pattern table from one row that holds
+// them (k_pat_table), and every row takes its id and compares its differences
+// with the pattern's, so that no hash decides (k_pat_ids).
+constexpr int kPatSlots = 1024;
+struct PatWork {
+  int32_t n, fail;
+  unsigned long long key[kPatSlots];  // 0: empty
+  int32_t row[kPatSlots], id[kPatSlots];
+};
+
+__global__ void k_pat_clear(PatWork *w) {
+  w->key[threadIdx.x] = 0;
+  if (threadIdx.x == 0) w->n = w->fail = 0;
+}
+
+__device__ __forceinline__ unsigned long long pat_hash(int64_t r, int32_t len,
+                                                       const int32_t *__restrict__ ci) {
+  unsigned long long h = 0x9e3779b97f4a7c15ull * (unsigned)(len + 1);
+  for (int32_t j = 0; j < len; j++) {
+    h = (h ^ (unsigned)(ci[j] - (int32_t)r)) * 0xff51afd7ed558ccdull;
+    h ^= h >> 32;
+  }
+  return h ? h : 1;
+}
+
+__global__ __launch_bounds__(kBlock) void k_pat_find(int64_t rows, const int32_t *__restrict__ rp,
+                                                     const int32_t *__restrict__ ci, PatWork *w,
+                                                     int32_t cap) {
+  const int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (r >= rows) return;
+  if (__hip_atomic_load(&w->fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+  const int32_t ra = rp[r];
+  const unsigned long long h = pat_hash(r, rp[r + 1] - ra, ci + ra);
+  // (at most cap of the slots fill before `fail` stops the search: an empty
+  // one is always met)
+  for (int k = 0; k < kPatSlots; k++) {
+    const int at = (int)((h + (unsigned)k) % kPatSlots);
+    unsigned long long have =
+        __hip_atomic_load(&w->key[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (have == 0) {
+      have = atomicCAS(&w->key[at], 0ull, h);
+      if (have == 0) {
+        w->row[at] = (int32_t)r;
+        if (atomicAdd(&w->n, 1) >= cap) atomicExch(&w->fail, 1);
+        return;
+      }
+    }
+    if (have == h) return;
+  }
+  atomicExch(&w->fail, 1);
+}
+
+__global__ __launch_bounds__(kPatSlots) void k_pat_table(const int32_t *__restrict__ rp,
+                                                         const int32_t *__restrict__ ci,
+                                                         PatWork *w, int32_t cap, int32_t stride,
+                                                         int32_t *tab) {
+  __shared__ int next;
+  if (w->fail) return;
+  if (threadIdx.x == 0) next = 0;
+  __syncthreads();
+  if (w->key[threadIdx.x] == 0) return;
+  const int id = atomicAdd(&next, 1);
+  w->id[threadIdx.x] = id;
+  if (id >= cap) return;
+  const int32_t r = w->row[threadIdx.x], ra = rp[r], len = min(rp[r + 1] - ra, stride - kPatHead);
+  int32_t *const t = tab + (int64_t)id * stride;
+  for (int j = 0; j < stride; j++)
+    t[j] = j == 0 ? len : j < kPatHead || j - kPatHead >= len ? 0 : ci[ra + j - kPatHead] - r;
+}
+
+__global__ __launch_bounds__(kBlock) void k_pat_ids(int64_t rows, const int32_t *__restrict__ rp,
+                                                    const int32_t *__restrict__ ci, PatWork *w,
+                                                    int32_t cap, int32_t stride,
+                                                    const int32_t *__restrict__ tab,
+                                                    uint8_t *pat) {
+  const int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (r >= rows || w->fail) return;
+  const int32_t ra = rp[r], len = rp[r + 1] - ra;
+  const unsigned long long h = pat_hash(r, len, ci + ra);
+  int id = -1;
+  for (int k = 0; k < kPatSlots && id < 0; k++) {
+    const int at = (int)((h + (unsigned)k) % kPatSlots);
+    if (w->key[at] == h) id = w->id[at];
+    else if (w->key[at] == 0) break;
+  }
+  bool ok = id >= 0 && id < cap;
+  const int32_t *const t = tab + (int64_t)(ok ? id : 0) * stride;
+  ok = ok && t[0] == len;
+  for (int32_t j = 0; ok && j < len; j++) ok = t[kPatHead + j] == ci[ra + j] - (int32_t)r;
+  if (!ok) atomicExch(&w->fail, 1);
+  pat[r] = (uint8_t)(ok ? id : 0);
+}
+
 // q = A p in the sliced layout for a matrix without long rows, one block of
 // 512 lanes per 512-row tile (a lane per row, as k_spmv_sell), and the tile
 // partial of <p, q> exactly as the CG engine's split-form kernels form it
@@ -244,12 +345,15 @@ __global__ void k_sell_fill(int64_t rows, const int32_t *__restrict__ rp,
 // 27-point stencil.  R: the partials' type (double with FP32 values for the
 // mixed-precision solver, whose products and sums are then exact-ish);
 // dcorr (or nullptr) adds a per-row diagonal correction after the row sum.
-template <class T, int W, class R>
+// PAT: the columns come from the row patterns (mgx_sell.hpp).
+template <class T, int W, class R, bool PAT>
 __global__ __launch_bounds__(kTile) void k_spmv_sell_pq(
     int64_t rows, int64_t ntiles, const int32_t *__restrict__ rp,
     const uint8_t *__restrict__ slen, const int64_t *__restrict__ soff,
     const int32_t *__restrict__ sci, const T *__restrict__ sval, const T *__restrict__ p,
-    T *__restrict__ q, R *P, const T *__restrict__ dcorr, int remap, const int32_t *live) {
+    T *__restrict__ q, R *P, const T *__restrict__ dcorr, int remap, const int32_t *live,
+    SellPat pt) {
+  extern __shared__ __align__(16) int32_t pat_lds[];
   __shared__ T qs[kTile];
   __shared__ R sh[kTile / 64];
   const int64_t tile = xcd_block(remap);
@@ -259,7 +363,17 @@ __global__ __launch_bounds__(kTile) void k_spmv_sell_pq(
   static_assert(kTile == 2 * kBlock, "the partial pairs rows of a 512-row tile");
   {
     const int64_t r = r0 + threadIdx.x;
-    const int32_t len = r < rows ? sell_len<T>(slen, rp, r) : 0;
+    int32_t len;
+    const int32_t *off = nullptr;
+    if constexpr (PAT) {
+      const int32_t id = r < rows ? pt.id[r] : 0;
+      sell_pat_stage(pt, pat_lds);
+      __syncthreads();
+      off = pat_lds + id * pt.stride;
+      len = r < rows ? off[0] : 0;
+    } else {
+      len = r < rows ? sell_len<T>(slen, rp, r) : 0;
+    }
     // the correction's two loads are issued before the row's gathers
     T dc = 0, pr = 0;
     if (dcorr && r < rows) {
@@ -267,7 +381,14 @@ __global__ __launch_bounds__(kTile) void k_spmv_sell_pq(
       pr = p[r];
     }
     T s = 0;
-    if (len) s = sell_row<T, W>(r, len, soff, sci, sval, [p](int64_t c) { return p[c]; });
+    if constexpr (PAT) {
+      const int64_t sl = 2 * wave_slice(r);
+      if (len)
+        s = sell_row_pat<T, W>(r, len, soff[sl], soff[sl + 1], off + kPatHead, sval,
+                               [p](int64_t c) { return p[c]; });
+    } else if (len) {
+      s = sell_row<T, W>(r, len, soff, sci, sval, [p](int64_t c) { return p[c]; });
+    }
     if (dcorr && r < rows) s = s + dc * pr;
     if (r < rows) q[r] = s;
     qs[threadIdx.x] = s;
@@ -289,20 +410,33 @@ __global__ __launch_bounds__(kTile) void k_spmv_sell_pq(
   if (threadIdx.x == 0) publish_partial(P, tile, t);
 }
 
-template <class T, bool AB, int W>
+template <class T, bool AB, int W, bool PAT>
 __global__ __launch_bounds__(kBlock) void k_spmv_sell(
     int64_t rows, int64_t nblocks, const int32_t *__restrict__ rp,
     const uint8_t *__restrict__ slen, const int64_t *__restrict__ soff,
     const int32_t *__restrict__ sci, const T *__restrict__ sval, const T *__restrict__ x,
-    T *__restrict__ y, T alpha, T beta, int long_t, int remap, const int32_t *live) {
+    T *__restrict__ y, T alpha, T beta, int long_t, int remap, const int32_t *live, SellPat pt) {
+  extern __shared__ __align__(16) int32_t pat_lds[];
   const int64_t b = xcd_block(remap);
   if (b >= nblocks) return;
   if (live && *live != kStatRunning) return;
   const int64_t r = b * kBlock + threadIdx.x;
-  if (r >= rows) return;
-  const int32_t len = sell_len<T>(slen, rp, r);
-  if (len > long_t) return;  // a long row: k_spmv_longrows
-  const T s = sell_row<T, W>(r, len, soff, sci, sval, [x](int64_t c) { return x[c]; });
+  T s;
+  if constexpr (PAT) {  // (no long rows)
+    const int32_t id = r < rows ? pt.id[r] : 0;
+    sell_pat_stage(pt, pat_lds);
+    __syncthreads();
+    if (r >= rows) return;
+    const int32_t *const off = pat_lds + id * pt.stride;
+    const int64_t sl = 2 * wave_slice(r);
+    s = sell_row_pat<T, W>(r, off[0], soff[sl], soff[sl + 1], off + kPatHead, sval,
+                           [x](int64_t c) { return x[c]; });
+  } else {
+    if (r >= rows) return;
+    const int32_t len = sell_len<T>(slen, rp, r);
+    if (len > long_t) return;  // a long row: k_spmv_longrows
+    s = sell_row<T, W>(r, len, soff, sci, sval, [x](int64_t c) { return x[c]; });
+  }
   if (AB) {
     T t = alpha * s;
     if (beta != T(0)) {
@@ -514,7 +648,60 @@ static void sliced_free(SpmvPlan::Sliced &l) {
   dev_free(l.d_sci);
   dev_free(l.d_val);
   dev_free(l.d_len);
+  dev_free(l.d_pat);
+  dev_free(l.d_ptab);
   l = SpmvPlan::Sliced();
+}
+
+// Row patterns of a layout (mgx_sell.hpp), looked for when the layout is
+// made.  From kPatNnz entries on: an SpMV of fewer takes some 4 us, most of it
+// latency, to which staging the table adds (sliced without / with patterns:
+// 5-point FP64, 0.33 M entries 3.5 / 3.8 us, 1.3 M 4.3 / 4.1 us in FP64 and
+// 3.8 / 3.9 us in FP32; 7-point, 1.8 M 4.9 / 4.9 us and 4.4 / 3.8 us).  A
+// matrix with more patterns than the table holds is given up by the rows that
+// start after the table has filled.
+constexpr int64_t kPatNnz = 3 << 19;
+
+static void sliced_patterns(Csr *A, SpmvPlan::Sliced &l) {
+  Ctx *c = A->ctx;
+  const int32_t maxr = A->plan.max_row;
+  const int32_t stride = kPatHead + (maxr + 3) / 4 * 4;
+  if (A->nnz < kPatNnz || maxr < 1 || 2 * stride > kPatWords) return;
+  const int32_t cap = std::min<int32_t>(kPatMax, kPatWords / stride);
+  void *w = nullptr;
+  try {
+    w = dev_alloc(sizeof(PatWork));
+    l.d_pat = (uint8_t *)dev_alloc((size_t)A->rows + 16);
+    l.d_ptab = (int32_t *)dev_alloc((size_t)cap * stride * 4);
+    PatWork *const pw = static_cast<PatWork *>(w);
+    const unsigned g = (unsigned)((A->rows + kBlock - 1) / kBlock);
+    k_pat_clear<<<1, kPatSlots, 0, c->stream>>>(pw);
+    k_pat_find<<<g, kBlock, 0, c->stream>>>(A->rows, A->rp, A->ci, pw, cap);
+    k_pat_table<<<1, kPatSlots, 0, c->stream>>>(A->rp, A->ci, pw, cap, stride, l.d_ptab);
+    k_pat_ids<<<g, kBlock, 0, c->stream>>>(A->rows, A->rp, A->ci, pw, cap, stride, l.d_ptab,
+                                           l.d_pat);
+    MGX_HIP(hipGetLastError());
+    int32_t res[2];
+    MGX_HIP(hipMemcpyAsync(res, &pw->n, sizeof res, hipMemcpyDeviceToHost, c->stream));
+    MGX_HIP(hipStreamSynchronize(c->stream));
+    if (res[1] == 0 && res[0] <= cap) {
+      l.npat = res[0];
+      l.pstride = stride;
+    }
+  } catch (const Error &e) {  // (without memory for them: the columns serve)
+    if (e.code != MGX_ERR_NOMEM) {
+      dev_free(w);
+      throw;
+    }
+    (void)hipGetLastError();
+  }
+  dev_free(w);
+  if (l.npat == 0) {
+    dev_free(l.d_pat);
+    dev_free(l.d_ptab);
+    l.d_pat = nullptr;
+    l.d_ptab = nullptr;
+  }
 }
 
 double sample_gather_lines(const int32_t *ci, int64_t nnz, size_t es) {
@@ -610,6 +797,7 @@ static void sliced_fill(Csr *A, SpmvPlan::Sliced &l, const std::vector<int64_t> 
                                                  l.d_len);
   MGX_HIP(hipGetLastError());
   MGX_HIP(hipStreamSynchronize(c->stream));
+  sliced_patterns(A, l);
 }
 
 template <class T, int W>
@@ -1056,6 +1244,11 @@ static void spmv_panels_dispatch(Csr *A, const T *X, T *Y) {
   MGX_HIP(hipGetLastError());
 }
 
+static SellPat sell_pat(const SpmvPlan::Sliced &l) {
+  return SellPat{l.d_pat, l.d_ptab, l.npat, l.pstride};
+}
+static size_t pat_bytes(const SellPat &pt) { return (size_t)pt.n * pt.stride * 4; }
+
 template <class T, bool AB>
 static void spmv_sell_dispatch(Csr *A, const SpmvPlan::Sliced &l, const T *V, const T *X, T *Y,
                                T alpha, T beta, const int32_t *live) {
@@ -1066,9 +1259,12 @@ static void spmv_sell_dispatch(Csr *A, const SpmvPlan::Sliced &l, const T *V, co
   const int remap = rg.remap;
   const unsigned grid = rg.grid;
   constexpr int W = sizeof(T) == 8 ? 2 : 4;
-  k_spmv_sell<T, AB, W><<<grid, kBlock, 0, c->stream>>>(
+  const SellPat pt = sell_pat(l);
+  const auto k = pt.n && p.nslong == 0 ? &k_spmv_sell<T, AB, W, true>
+                                       : &k_spmv_sell<T, AB, W, false>;
+  k<<<grid, kBlock, pt.n && p.nslong == 0 ? pat_bytes(pt) : 0, c->stream>>>(
       A->rows, nb, A->rp, l.d_len, l.d_soff, l.d_sci, static_cast<const T *>(l.d_val), X, Y,
-      alpha, beta, p.long_row, remap, live);
+      alpha, beta, p.long_row, remap, live, pt);
   if (p.nslong > 0)
     k_spmv_longrows<T, AB><<<(unsigned)p.nslong, kBlock, 0, c->stream>>>(
         p.d_slrows, p.nslong, A->rp, A->ci, V, X, Y, alpha, beta, live);
@@ -1469,22 +1665,24 @@ bool spmv_sell_pq(Csr *A, const void *val, mgx_dtype dt, const void *p, void *q,
   const RemapGrid rg = remap_grid(A->plan.remap, nt);
   const int remap = rg.remap;
   const unsigned grid = rg.grid;
+  const SellPat pt = sell_pat(*l);
+  const auto run = [&](auto k, auto tv, auto pv) {
+    using T = decltype(tv);
+    using R = decltype(pv);
+    k<<<grid, kTile, pat_bytes(pt), c->stream>>>(
+        A->rows, nt, A->rp, l->d_len, l->d_soff, l->d_sci, static_cast<const T *>(l->d_val),
+        static_cast<const T *>(p), static_cast<T *>(q), static_cast<R *>(P),
+        acc64 ? reinterpret_cast<const T *>(dcorr) : nullptr, remap, live, pt);
+  };
   if (dt == MGX_F64)
-    k_spmv_sell_pq<double, 2, double><<<grid, kTile, 0, c->stream>>>(
-        A->rows, nt, A->rp, l->d_len, l->d_soff, l->d_sci,
-        static_cast<const double *>(l->d_val),
-        static_cast<const double *>(p), static_cast<double *>(q), static_cast<double *>(P),
-        nullptr, remap, live);
+    run(pt.n ? &k_spmv_sell_pq<double, 2, double, true>
+             : &k_spmv_sell_pq<double, 2, double, false>, double(), double());
   else if (acc64)
-    k_spmv_sell_pq<float, 4, double><<<grid, kTile, 0, c->stream>>>(
-        A->rows, nt, A->rp, l->d_len, l->d_soff, l->d_sci, static_cast<const float *>(l->d_val),
-        static_cast<const float *>(p), static_cast<float *>(q), static_cast<double *>(P), dcorr,
-        remap, live);
+    run(pt.n ? &k_spmv_sell_pq<float, 4, double, true>
+             : &k_spmv_sell_pq<float, 4, double, false>, float(), double());
   else
-    k_spmv_sell_pq<float, 4, float><<<grid, kTile, 0, c->stream>>>(
-        A->rows, nt, A->rp, l->d_len, l->d_soff, l->d_sci, static_cast<const float *>(l->d_val),
-        static_cast<const float *>(p), static_cast<float *>(q), static_cast<float *>(P), nullptr,
-        remap, live);
+    run(pt.n ? &k_spmv_sell_pq<float, 4, float, true>
+             : &k_spmv_sell_pq<float, 4, float, false>, float(), float());
   MGX_HIP(hipGetLastError());
   return true;
 }

@@ -606,6 +606,63 @@ def test_matvec_sliced_layout(m, ctx, oracle, dtype):
         assert bits_equal(xs[0], xs[1])
 
 
+def pattern_rows(rng, rows, npat, lens, span):
+    """A matrix of `rows` rows that take turns at npat lists of column - row
+    differences in [0, span), as many as lens gives in turn."""
+    lists = [np.sort(rng.choice(span, lens[k % len(lens)], replace=False))
+             for k in range(npat)]
+    which = np.arange(rows) % npat
+    which[:64] = np.arange(64) % min(npat, 3)
+    ln = np.array([len(l) for l in lists])[which]
+    rp = np.zeros(rows + 1, np.int32)
+    np.cumsum(ln, out=rp[1:])
+    ci = np.concatenate([lists[w] + r for r, w in enumerate(which)]) if rp[-1] else []
+    return rp, np.asarray(ci, np.int32), rows + span
+
+
+@pytest.mark.parametrize("rows,npat,lens,span", [
+    (174763, 1, (9,), 40),           # 3 * 2^19 + 3 entries; the last slice partly full
+    (174762, 3, (9, 9, 9), 40),      # 6 entries over the line
+    (174761, 3, (9, 9, 9), 40),      # below it: columns from memory
+    (140001, 255, (12, 11, 12, 10), 64),
+    (140001, 256, (12, 11, 12, 10), 64),  # one pattern too many
+    (140003, 300, (12, 11), 64),
+    (120001, 5, (16, 15, 14, 13), 3000),
+    (520000, 7, (3, 4, 4, 3), 12),   # rows of tail entries only, or one tuple
+    (40001, 9, (60, 59, 58, 57), 90),
+    (70001, 60, (64, 63, 61), 90),   # 60 * 68 words fill the table
+    (70001, 61, (64, 63, 61), 90),   # and 61 do not fit it
+])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_sliced_row_patterns(m, ctx, oracle, dtype, rows, npat, lens, span):
+    """The sliced layout with the columns from row patterns: the CPU row
+    loop's bits, on both sides of the entry count from which patterns are
+    looked for, of the most patterns and the most table words held, for
+    remainders of the tuples; new values go through the same patterns."""
+    say("sliced row patterns", dtype.__name__, rows, npat)
+    rng = np.random.default_rng(rows + npat)
+    rp, ci, cols = pattern_rows(rng, rows, npat, lens, span)
+    val = rng.uniform(-1, 1, rp[-1]).astype(dtype)
+    x = oracle.random_vector(cols, -1.0, 1.0, 40, dtype=dtype)
+    y0 = oracle.random_vector(rows, -1.0, 1.0, 41, dtype=dtype)
+    A = m.CRS(ctx, rows, cols, rp, ci, val)
+    X, Y = m.Vector(ctx, x, dtype=dtype), m.Vector(ctx, y0, dtype=dtype)
+    m.matvec_ab(0.5, A, X, -2.0, Y)
+    ab = Y.download()
+    A.set_plan(row_walk=2)
+    m.matvec(A, X, Y)
+    assert bits_equal(Y.download(), oracle.spmv(rp, ci, val, x))
+    Y.upload(y0)
+    m.matvec_ab(0.5, A, X, -2.0, Y)
+    assert bits_equal(Y.download(), ab)
+    v2 = (val * 3).astype(dtype)
+    A.update_values(v2)
+    m.matvec(A, X, Y)
+    assert bits_equal(Y.download(), oracle.spmv(rp, ci, v2, x))
+    for o in (A, X, Y):
+        o.free()
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_dot_nrm2_device_results(m, ctx, oracle, dtype):
     """mgx_dot_device / mgx_nrm2_device leave the result in device memory:
