@@ -95,7 +95,10 @@ typedef struct mgx_spmv_tuning {
   double us;           /* time of one SpMV under the chosen plan */
   int32_t candidates;  /* plans timed */
   int32_t column_panels; /* 0, or the column panels of the chosen plan */
-  int32_t row_walk;    /* 0 products staged in LDS in entry order; 1 row
+  int32_t row_walk;    /* 0 products staged in LDS in entry order (a large
+                          matrix whose rows hold few distinct lists of
+                          column - row: values staged, a lane per row, in
+                          blocks of the library's choice); 1 row
                           walk (lane per row over LDS-staged val / col_ind;
                           coalesced gathers on banded rows); 2 the sliced
                           layout; 3 L2 panels (row sums kept in LDS while the

@@ -171,6 +171,8 @@ struct SpmvPlan {
                          // c > 1 runs of c blocks dealt to the XCDs in turn
   int32_t walk = 0;      // stream blocks: 0 product-staged, 1 row walk
   double mean_row = 0;
+  int32_t rowpat = 0;    // block plan of a matrix with row patterns: values
+                         // staged, columns from the patterns (walk unused)
   double tuned_us = 0;   // SpMV time measured by the autotuner (0: not tuned)
   // column-panel mode (0: off): the short rows' entries are also stored
   // panel-major (panel k holds columns [k*pwidth, (k+1)*pwidth)), each pass
@@ -198,11 +200,6 @@ struct SpmvPlan {
     // row lengths, min(len, 255): the kernels read row_ptr only for rows
     // of 255 entries or more
     uint8_t *d_len = nullptr;
-    // row patterns (mgx_sell.hpp), where the matrix has few enough: a byte
-    // per row and the table (npat 0: none)
-    uint8_t *d_pat = nullptr;
-    int32_t *d_ptab = nullptr;
-    int32_t npat = 0, pstride = 0;
   };
   int32_t sell = 0;
   Sliced sl, sl32;
@@ -237,6 +234,13 @@ struct Csr {
   void *val = nullptr;
   std::vector<int32_t> rp_raw;  // kept only when it differs from rp
   SpmvPlan plan;
+  // row patterns (mgx_sell.hpp), where the matrix has few enough (npat 0:
+  // none): a byte per row (in col_ind's allocation, nullptr without room),
+  // the table; looked for once, with the first plan
+  uint8_t *d_pat = nullptr;
+  int32_t *d_ptab = nullptr;
+  int32_t npat = 0, pstride = 0;
+  bool pat_done = false;
   // fused-solver plan: row chunks that never cross a 512-row tile; the sign
   // bit marks a long row; tile k owns chunks [tile_chunk[k], tile_chunk[k+1])
   int32_t *d_chunks = nullptr;
@@ -384,6 +388,8 @@ struct LpanelLayout {
 bool lpanel_layout(const int32_t *rp, const int32_t *ci, const char *val, size_t es, int64_t n,
                    int64_t cols, int long_t, int npanels, LpanelLayout &L);
 void spmv_sell_free(Csr *A);
+size_t spmv_patterns_room(const Csr *A, int64_t nnz);  // bytes behind col_ind
+bool spmv_rowpat_ok(const Csr *A);  // plan.rowpat may be set
 void spmv_sell_values(Csr *A);  // refresh the sliced values after a change
 void launch_diag_v(Csr *A, const void *val, mgx_dtype dt, void *d);
 // fused-solver row chunks (built at upload for square matrices, from the

@@ -132,7 +132,18 @@ static bool overlap(const Vec *a, const Vec *b) {
 constexpr int64_t kEntryPad = 4;
 void alloc_entries(Csr *A, int64_t nnz) {
   const size_t cnt = (size_t)(std::max<int64_t>(nnz, 0) + kEntryPad);
-  A->ci = (int32_t *)dev_alloc(cnt * 4);
+  // room for the row patterns behind col_ind (an allocation of its own took
+  // 0.15 ms of every upload and destruction); without memory for it there are
+  // no patterns
+  const size_t at = (cnt * 4 + 255) / 256 * 256, room = spmv_patterns_room(A, nnz);
+  try {
+    A->ci = (int32_t *)dev_alloc(room ? at + room : cnt * 4);
+    A->d_pat = room ? (uint8_t *)A->ci + at : nullptr;
+  } catch (const Error &e) {
+    if (!room || e.code != MGX_ERR_NOMEM) throw;
+    (void)hipGetLastError();
+    A->ci = (int32_t *)dev_alloc(cnt * 4);
+  }
   A->val = dev_alloc(cnt * A->elem());
   MGX_HIP(hipMemsetAsync(A->ci + nnz, 0, kEntryPad * 4, A->ctx->stream));
   MGX_HIP(hipMemsetAsync((char *)A->val + nnz * A->elem(), 0, kEntryPad * A->elem(),
@@ -342,6 +353,7 @@ int mgx_csr_set_plan(mgx_csr *A, int rows_per_block, int nnz_per_block, int xcd_
                 "mgx_csr_set_plan: the sliced layout and column panels exclude each other");
     spmv_plan_build_with(A, rp.data(), rows_per_block, nnz_per_block, long_t, xcd_remap,
                          row_walk == 1);
+    if (row_walk == 0 && !column_panels) A->plan.rowpat = spmv_rowpat_ok(A);
     if (row_walk == 3)
       MGX_REQUIRE(spmv_lpanel_build(A, column_panels),
                   "mgx_csr_set_plan: L2 panels need ascending columns within rows and at "

@@ -241,7 +241,10 @@ __device__ __forceinline__ int64_t wave_slice(int64_t r) {
 }
 
 // Finding the row patterns: rows enter a 64-bit hash of their differences
-// into a small open table (k_pat_find; a row that finds more than cap of them
+// into a small open table (k_pat_find: one block takes kPatSlots rows spread
+// over the matrix first, so that a matrix with many patterns fails there and
+// the other rows find theirs entered, instead of half a million of them
+// contending for the first entry; a row that finds more than cap of them
 // raises `fail`, and the rows after it return at once), the table's entries
 // get their ids and their row of the pattern table from one row that holds
 // them (k_pat_table), and every row takes its id and compares its differences
@@ -268,17 +271,20 @@ __device__ __forceinline__ unsigned long long pat_hash(int64_t r, int32_t len,
   return h ? h : 1;
 }
 
-__global__ __launch_bounds__(kBlock) void k_pat_find(int64_t rows, const int32_t *__restrict__ rp,
-                                                     const int32_t *__restrict__ ci, PatWork *w,
-                                                     int32_t cap) {
-  const int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+constexpr int kPatProbes = 32;  // a quarter of the slots is used at most
+
+// row blockIdx.x * blockDim.x + threadIdx.x, or that of `of` equal steps
+__global__ __launch_bounds__(kPatSlots) void k_pat_find(int64_t rows,
+                                                        const int32_t *__restrict__ rp,
+                                                        const int32_t *__restrict__ ci,
+                                                        PatWork *w, int32_t cap, int64_t of) {
+  int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (of) r = r * rows / of;
   if (r >= rows) return;
   if (__hip_atomic_load(&w->fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
   const int32_t ra = rp[r];
   const unsigned long long h = pat_hash(r, rp[r + 1] - ra, ci + ra);
-  // (at most cap of the slots fill before `fail` stops the search: an empty
-  // one is always met)
-  for (int k = 0; k < kPatSlots; k++) {
+  for (int k = 0; k < kPatProbes; k++) {
     const int at = (int)((h + (unsigned)k) % kPatSlots);
     unsigned long long have =
         __hip_atomic_load(&w->key[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -323,7 +329,7 @@ __global__ __launch_bounds__(kBlock) void k_pat_ids(int64_t rows, const int32_t 
   const int32_t ra = rp[r], len = rp[r + 1] - ra;
   const unsigned long long h = pat_hash(r, len, ci + ra);
   int id = -1;
-  for (int k = 0; k < kPatSlots && id < 0; k++) {
+  for (int k = 0; k < kPatProbes && id < 0; k++) {
     const int at = (int)((h + (unsigned)k) % kPatSlots);
     if (w->key[at] == h) id = w->id[at];
     else if (w->key[at] == 0) break;
@@ -444,6 +450,76 @@ __global__ __launch_bounds__(kBlock) void k_spmv_sell(
       t = t + u;
     }
     y[r] = t;
+  } else {
+    y[r] = s;
+  }
+}
+
+// A block plan's SpMV of a matrix with row patterns and without long rows: a
+// block stages the values of its blockDim.x rows in LDS (one run of the CRS
+// array, whole 16-byte loads; the array is padded) and each lane walks its
+// row there, the columns from the patterns, so no copy of the matrix is
+// needed.  Bound by the values it streams.  Products staged with columns from
+// memory / this (us): 7-point 192^3 FP64 147 / 89, FP32 91 / 54; 27-point
+// 128^3 145 / 112 and 99 / 52; 5-point 1000^2 16.2 / 11.6 and 11.3 / 8.0; rows
+// of 12 entries, 1 M rows, 32 / 23 and 20 / 12; of 16 (bank conflicts at
+// their worst) 42 / 30 and 25 / 21.
+template <class T, bool AB>
+__global__ __launch_bounds__(kBlock) void k_spmv_pat(
+    int64_t rows, int64_t nblocks, const int32_t *__restrict__ rp, const T *__restrict__ val,
+    const T *__restrict__ x, T *__restrict__ y, T alpha, T beta, int remap, const int32_t *live,
+    SellPat pt) {
+  constexpr int W = 16 / (int)sizeof(T), G = 8;
+  typedef T VT __attribute__((ext_vector_type(W)));
+  extern __shared__ __align__(16) int32_t pat_lds[];
+  T *const sv = reinterpret_cast<T *>(pat_lds + pt.n * pt.stride);
+  const int64_t b = xcd_block(remap);
+  if (b >= nblocks) return;
+  if (live && *live != kStatRunning) return;
+  const int nth = (int)blockDim.x, t = (int)threadIdx.x;
+  const int64_t r0 = b * nth, r = r0 + t, rc = r < rows ? r : rows - 1;
+  const int32_t e0 = rp[r0], e1 = rp[r0 + nth < rows ? r0 + nth : rows];
+  const int32_t ea = e0 & ~(W - 1);
+  const int32_t id = pt.id[rc], ra = rp[rc];
+  for (int32_t k0 = ea + t * W; k0 < e1; k0 += G * nth * W) {
+    VT v[G];
+#pragma unroll
+    for (int k = 0; k < G; k++)
+      if (k0 + k * nth * W < e1)
+        v[k] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(val + k0 + k * nth * W));
+#pragma unroll
+    for (int k = 0; k < G; k++)
+      if (k0 + k * nth * W < e1) *reinterpret_cast<VT *>(sv + (k0 - ea) + k * nth * W) = v[k];
+  }
+  sell_pat_stage(pt, pat_lds);
+  __syncthreads();
+  if (r >= rows) return;
+  const int32_t *const row = pat_lds + id * pt.stride, *const off = row + kPatHead;
+  const int32_t len = row[0];
+  const T *const w = sv + (ra - ea);
+  T s = 0;
+  for (int32_t j = 0; j < len; j += 8) {
+    T vv[8], xv[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (j + q < len) {
+        xv[q] = x[(int32_t)r + off[j + q]];
+        vv[q] = w[j + q];
+      }
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (j + q < len) {
+        T p = vv[q] * xv[q];
+        s = s + p;
+      }
+  }
+  if (AB) {
+    T u = alpha * s;
+    if (beta != T(0)) {
+      T w2 = beta * y[r];
+      u = u + w2;
+    }
+    y[r] = u;
   } else {
     y[r] = s;
   }
@@ -583,8 +659,78 @@ __global__ __launch_bounds__(kBlock) void k_diag(int64_t n, const int32_t *__res
 
 }  // namespace
 
+// Row patterns (mgx_sell.hpp), looked for when the first plan is made: from
+// kPatNnz entries on.  An SpMV of fewer takes some 4 us, most of it latency,
+// to which staging the table adds (sliced without / with patterns: 5-point
+// FP64, 0.33 M entries 3.5 / 3.8 us, 1.3 M 4.3 / 4.1 us in FP64 and 3.8 / 3.9
+// us in FP32; 7-point, 1.8 M 4.9 / 4.9 us and 4.4 / 3.8 us).  A matrix with
+// more patterns than the table holds is given up early; without memory for
+// the patterns the columns serve.
+constexpr int64_t kPatNnz = 3 << 19;
+
+static size_t pat_ids_bytes(const Csr *A) { return ((size_t)A->rows + 255) / 256 * 256; }
+
+// ids, table, and what only the search needs
+size_t spmv_patterns_room(const Csr *A, int64_t nnz) {
+  return nnz < kPatNnz ? 0 : pat_ids_bytes(A) + (size_t)kPatWords * 4 + sizeof(PatWork);
+}
+
+static void spmv_patterns(Csr *A) {
+  if (A->pat_done) return;
+  A->pat_done = true;
+  Ctx *c = A->ctx;
+  const int32_t maxr = A->plan.max_row;
+  const int32_t stride = kPatHead + (maxr + 3) / 4 * 4;
+  if (!A->d_pat || maxr < 1 || 2 * stride > kPatWords) return;
+  const int32_t cap = std::min<int32_t>(kPatMax, kPatWords / stride);
+  A->d_ptab = (int32_t *)(A->d_pat + pat_ids_bytes(A));
+  PatWork *const pw = (PatWork *)(A->d_ptab + kPatWords);
+  const unsigned g = (unsigned)((A->rows + kBlock - 1) / kBlock);
+  k_pat_clear<<<1, kPatSlots, 0, c->stream>>>(pw);
+  k_pat_find<<<1, kPatSlots, 0, c->stream>>>(A->rows, A->rp, A->ci, pw, cap, kPatSlots);
+  k_pat_find<<<g, kBlock, 0, c->stream>>>(A->rows, A->rp, A->ci, pw, cap, 0);
+  k_pat_table<<<1, kPatSlots, 0, c->stream>>>(A->rp, A->ci, pw, cap, stride, A->d_ptab);
+  k_pat_ids<<<g, kBlock, 0, c->stream>>>(A->rows, A->rp, A->ci, pw, cap, stride, A->d_ptab,
+                                         A->d_pat);
+  MGX_HIP(hipGetLastError());
+  int32_t res[2];
+  MGX_HIP(hipMemcpyAsync(res, &pw->n, sizeof res, hipMemcpyDeviceToHost, c->stream));
+  MGX_HIP(hipStreamSynchronize(c->stream));
+  if (res[1] == 0 && res[0] <= cap) {
+    A->npat = res[0];
+    A->pstride = stride;
+  }
+}
+
+static SellPat sell_pat(const Csr *A) {
+  return SellPat{A->d_pat, A->d_ptab, A->npat, A->pstride};
+}
+static size_t pat_bytes(const SellPat &pt) { return (size_t)pt.n * pt.stride * 4; }
+
+// LDS of a k_spmv_pat block of `rows` rows, values of es bytes
+static size_t rowpat_bytes(const Csr *A, int rows, size_t es) {
+  return pat_bytes(sell_pat(A)) + ((size_t)rows * A->plan.max_row + 32 / es) * es;
+}
+
+// rows of a k_spmv_pat block: kBlock, or half of that where it would take more
+// than 32 KB of LDS and leave a compute unit few wavefronts (27-point 128^3
+// FP64, 59 KB: 118 us with 256 rows, 112 with 128; 16 entries a row, 33 KB:
+// 31.5 / 30.2; 27-point FP32, 31 KB: 52 / 58); 0: not even that fits, or the
+// lanes' rows start in the same bank (rows of 32 entries, FP64: products
+// staged 94.7, this 100.3)
+static int rowpat_rows(const Csr *A, size_t es) {
+  if (A->plan.max_row % 32 == 0) return 0;
+  if (rowpat_bytes(A, kBlock, es) <= 32768) return kBlock;
+  return rowpat_bytes(A, kBlock / 2, es) <= 65536 ? kBlock / 2 : 0;
+}
+
+bool spmv_rowpat_ok(const Csr *A) {
+  return A->npat > 0 && A->plan.nlong == 0 && rowpat_rows(A, A->elem()) > 0;
+}
+
 void spmv_plan_build(Ctx *c, Csr *A, const int32_t *rp) {
   spmv_plan_build_with(A, rp, c->spmv_rows, c->spmv_nnz, c->spmv_long, c->xcd_remap, 0);
+  A->plan.rowpat = spmv_rowpat_ok(A);
 }
 
 void spmv_plan_build_with(Csr *A, const int32_t *rp, int rows_req, int nnz_req, int long_req,
@@ -636,10 +782,12 @@ void spmv_plan_build_with(Csr *A, const int32_t *rp, int rows_req, int nnz_req, 
   A->plan.remap = remap_req > 1 ? std::min(remap_req, kMaxRemapRun) : (remap_req ? 1 : 0);
   A->plan.walk = walk ? 1 : 0;
   A->plan.tuned_us = 0;
+  A->plan.rowpat = 0;
   if (A->plan.d_blocks) dev_free(A->plan.d_blocks);
   A->plan.d_blocks = (int2 *)dev_alloc(blk.size() * sizeof(int2));
   MGX_HIP(hipMemcpyAsync(A->plan.d_blocks, blk.data(), blk.size() * sizeof(int2),
                          hipMemcpyHostToDevice, c->stream));
+  spmv_patterns(A);
   MGX_HIP(hipStreamSynchronize(c->stream));
 }
 
@@ -648,60 +796,7 @@ static void sliced_free(SpmvPlan::Sliced &l) {
   dev_free(l.d_sci);
   dev_free(l.d_val);
   dev_free(l.d_len);
-  dev_free(l.d_pat);
-  dev_free(l.d_ptab);
   l = SpmvPlan::Sliced();
-}
-
-// Row patterns of a layout (mgx_sell.hpp), looked for when the layout is
-// made.  From kPatNnz entries on: an SpMV of fewer takes some 4 us, most of it
-// latency, to which staging the table adds (sliced without / with patterns:
-// 5-point FP64, 0.33 M entries 3.5 / 3.8 us, 1.3 M 4.3 / 4.1 us in FP64 and
-// 3.8 / 3.9 us in FP32; 7-point, 1.8 M 4.9 / 4.9 us and 4.4 / 3.8 us).  A
-// matrix with more patterns than the table holds is given up by the rows that
-// start after the table has filled.
-constexpr int64_t kPatNnz = 3 << 19;
-
-static void sliced_patterns(Csr *A, SpmvPlan::Sliced &l) {
-  Ctx *c = A->ctx;
-  const int32_t maxr = A->plan.max_row;
-  const int32_t stride = kPatHead + (maxr + 3) / 4 * 4;
-  if (A->nnz < kPatNnz || maxr < 1 || 2 * stride > kPatWords) return;
-  const int32_t cap = std::min<int32_t>(kPatMax, kPatWords / stride);
-  void *w = nullptr;
-  try {
-    w = dev_alloc(sizeof(PatWork));
-    l.d_pat = (uint8_t *)dev_alloc((size_t)A->rows + 16);
-    l.d_ptab = (int32_t *)dev_alloc((size_t)cap * stride * 4);
-    PatWork *const pw = static_cast<PatWork *>(w);
-    const unsigned g = (unsigned)((A->rows + kBlock - 1) / kBlock);
-    k_pat_clear<<<1, kPatSlots, 0, c->stream>>>(pw);
-    k_pat_find<<<g, kBlock, 0, c->stream>>>(A->rows, A->rp, A->ci, pw, cap);
-    k_pat_table<<<1, kPatSlots, 0, c->stream>>>(A->rp, A->ci, pw, cap, stride, l.d_ptab);
-    k_pat_ids<<<g, kBlock, 0, c->stream>>>(A->rows, A->rp, A->ci, pw, cap, stride, l.d_ptab,
-                                           l.d_pat);
-    MGX_HIP(hipGetLastError());
-    int32_t res[2];
-    MGX_HIP(hipMemcpyAsync(res, &pw->n, sizeof res, hipMemcpyDeviceToHost, c->stream));
-    MGX_HIP(hipStreamSynchronize(c->stream));
-    if (res[1] == 0 && res[0] <= cap) {
-      l.npat = res[0];
-      l.pstride = stride;
-    }
-  } catch (const Error &e) {  // (without memory for them: the columns serve)
-    if (e.code != MGX_ERR_NOMEM) {
-      dev_free(w);
-      throw;
-    }
-    (void)hipGetLastError();
-  }
-  dev_free(w);
-  if (l.npat == 0) {
-    dev_free(l.d_pat);
-    dev_free(l.d_ptab);
-    l.d_pat = nullptr;
-    l.d_ptab = nullptr;
-  }
 }
 
 double sample_gather_lines(const int32_t *ci, int64_t nnz, size_t es) {
@@ -797,7 +892,6 @@ static void sliced_fill(Csr *A, SpmvPlan::Sliced &l, const std::vector<int64_t> 
                                                  l.d_len);
   MGX_HIP(hipGetLastError());
   MGX_HIP(hipStreamSynchronize(c->stream));
-  sliced_patterns(A, l);
 }
 
 template <class T, int W>
@@ -1244,11 +1338,6 @@ static void spmv_panels_dispatch(Csr *A, const T *X, T *Y) {
   MGX_HIP(hipGetLastError());
 }
 
-static SellPat sell_pat(const SpmvPlan::Sliced &l) {
-  return SellPat{l.d_pat, l.d_ptab, l.npat, l.pstride};
-}
-static size_t pat_bytes(const SellPat &pt) { return (size_t)pt.n * pt.stride * 4; }
-
 template <class T, bool AB>
 static void spmv_sell_dispatch(Csr *A, const SpmvPlan::Sliced &l, const T *V, const T *X, T *Y,
                                T alpha, T beta, const int32_t *live) {
@@ -1259,7 +1348,7 @@ static void spmv_sell_dispatch(Csr *A, const SpmvPlan::Sliced &l, const T *V, co
   const int remap = rg.remap;
   const unsigned grid = rg.grid;
   constexpr int W = sizeof(T) == 8 ? 2 : 4;
-  const SellPat pt = sell_pat(l);
+  const SellPat pt = sell_pat(A);
   const auto k = pt.n && p.nslong == 0 ? &k_spmv_sell<T, AB, W, true>
                                        : &k_spmv_sell<T, AB, W, false>;
   k<<<grid, kBlock, pt.n && p.nslong == 0 ? pat_bytes(pt) : 0, c->stream>>>(
@@ -1303,6 +1392,17 @@ static void spmv_dispatch(Csr *A, const T *V, const T *X, T *Y, T alpha,
   // column-panel mode: plain y = A x with A's own values, outside solver loops
   if (!AB && !live && A->plan.npanels > 0 && V == static_cast<const T *>(A->val)) {
     spmv_panels_dispatch<T>(A, X, Y);
+    return;
+  }
+  if (A->plan.rowpat) {
+    const SellPat pt = sell_pat(A);
+    const int rb = rowpat_rows(A, sizeof(T));
+    const int64_t nb = (A->rows + rb - 1) / rb;
+    const RemapGrid rg = remap_grid(A->plan.remap, nb);
+    const size_t lds = rowpat_bytes(A, rb, sizeof(T));
+    k_spmv_pat<T, AB><<<rg.grid, rb, lds, c->stream>>>(A->rows, nb, A->rp, V, X, Y, alpha, beta,
+                                                       rg.remap, live, pt);
+    MGX_HIP(hipGetLastError());
     return;
   }
   const int64_t nb = A->plan.nblocks;
@@ -1597,11 +1697,40 @@ void spmv_autotune(Csr *A, int reps, mgx_spmv_tuning *out) {
           if (keep_lp) spmv_lpanel_build(A, keep_lp);
         }
       }
+      // the block plan with row patterns, where it is clearly the faster
+      if (spmv_rowpat_ok(A) && !best_panels && !lpanel_best) {
+        const int sell = A->plan.sell, remap = A->plan.remap;
+        int pat_remap = remap;
+        double pat_us = 1e300;
+        A->plan.sell = 0;
+        A->plan.rowpat = 1;
+        for (int rr : {0, 1, 16}) {
+          A->plan.remap = rr;
+          ncand++;
+          const double us = timed(reps);
+          if (us < pat_us) {
+            pat_us = us;
+            pat_remap = rr;
+          }
+        }
+        A->plan.sell = sell;
+        A->plan.rowpat = 0;
+        A->plan.remap = remap;
+        if (pat_us < 0.97 * best_us) {
+          best_us = pat_us;
+          spmv_sell_free(A);
+          best_sell = 0;
+          best.walk = 0;
+          A->plan.rowpat = 1;
+          A->plan.remap = pat_remap;
+        }
+      }
     } catch (...) {
       if (e0) (void)hipEventDestroy(e0);
       if (e1) (void)hipEventDestroy(e1);
       dev_free(x);
       dev_free(y);
+      A->plan.sell = A->plan.sl.d_soff != nullptr;
       spmv_sell_free(A);
       throw;
     }
@@ -1665,7 +1794,7 @@ bool spmv_sell_pq(Csr *A, const void *val, mgx_dtype dt, const void *p, void *q,
   const RemapGrid rg = remap_grid(A->plan.remap, nt);
   const int remap = rg.remap;
   const unsigned grid = rg.grid;
-  const SellPat pt = sell_pat(*l);
+  const SellPat pt = sell_pat(A);
   const auto run = [&](auto k, auto tv, auto pv) {
     using T = decltype(tv);
     using R = decltype(pv);

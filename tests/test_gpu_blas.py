@@ -632,11 +632,17 @@ def pattern_rows(rng, rows, npat, lens, span):
     (40001, 9, (60, 59, 58, 57), 90),
     (70001, 60, (64, 63, 61), 90),   # 60 * 68 words fill the table
     (70001, 61, (64, 63, 61), 90),   # and 61 do not fit it
+    (100001, 2, (16, 16), 40),       # FP64: 32 KB of LDS are not enough for 256 rows
+    (100127, 2, (15, 14), 40),       # and are for these
+    (100129, 3, (63, 62, 61), 90),   # FP64: 128 rows take just under 64 KB
+    (100130, 3, (64, 63, 62), 90),   # and just over
+    (60001, 4, (32, 31, 30), 90),    # rows 32 apart in LDS: columns from memory
 ])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_sliced_row_patterns(m, ctx, oracle, dtype, rows, npat, lens, span):
-    """The sliced layout with the columns from row patterns: the CPU row
-    loop's bits, on both sides of the entry count from which patterns are
+    """The block plan and the sliced layout with the columns from row
+    patterns, and the plan that the autotuner takes: the CPU row loop's bits,
+    on both sides of the entry count from which patterns are
     looked for, of the most patterns and the most table words held, for
     remainders of the tuples; new values go through the same patterns."""
     say("sliced row patterns", dtype.__name__, rows, npat)
@@ -647,19 +653,27 @@ def test_sliced_row_patterns(m, ctx, oracle, dtype, rows, npat, lens, span):
     y0 = oracle.random_vector(rows, -1.0, 1.0, 41, dtype=dtype)
     A = m.CRS(ctx, rows, cols, rp, ci, val)
     X, Y = m.Vector(ctx, x, dtype=dtype), m.Vector(ctx, y0, dtype=dtype)
+    A.set_plan(row_walk=1)  # columns from memory
     m.matvec_ab(0.5, A, X, -2.0, Y)
     ab = Y.download()
-    A.set_plan(row_walk=2)
-    m.matvec(A, X, Y)
-    assert bits_equal(Y.download(), oracle.spmv(rp, ci, val, x))
-    Y.upload(y0)
-    m.matvec_ab(0.5, A, X, -2.0, Y)
-    assert bits_equal(Y.download(), ab)
-    v2 = (val * 3).astype(dtype)
-    A.update_values(v2)
-    m.matvec(A, X, Y)
-    assert bits_equal(Y.download(), oracle.spmv(rp, ci, v2, x))
-    for o in (A, X, Y):
+    A.free()
+    for plan in ("block", "sliced", "tuned"):
+        A = m.CRS(ctx, rows, cols, rp, ci, val)
+        if plan == "sliced":
+            A.set_plan(row_walk=2)
+        elif plan == "tuned":
+            A.autotune(reps=2)
+        m.matvec(A, X, Y)
+        assert bits_equal(Y.download(), oracle.spmv(rp, ci, val, x)), plan
+        Y.upload(y0)
+        m.matvec_ab(0.5, A, X, -2.0, Y)
+        assert bits_equal(Y.download(), ab), plan
+        v2 = (val * 3).astype(dtype)
+        A.update_values(v2)
+        m.matvec(A, X, Y)
+        assert bits_equal(Y.download(), oracle.spmv(rp, ci, v2, x)), plan
+        A.free()
+    for o in (X, Y):
         o.free()
 
 
