@@ -520,10 +520,11 @@ template <class T> bool Engine<T>::run_resident(int slot) {
   }
   // a launch ends after this many iterations (a second or two); the host
   // looks at the state and launches again if the solve is still running
-  constexpr int64_t kPerLaunch = 1 << 17;
+  const int64_t per_launch = c_->res_iters;
+  MGX_REQUIRE(per_launch > 0, "resident solve: no iterations per launch");
   for (bool fresh = true;; fresh = false) {
     resident_launch<T>(c_, method_[slot], d_sys_ + slot, nt, csr_[slot]->plan.max_row, d_res_,
-                       d_stopped_, kPerLaunch);
+                       d_stopped_, per_launch);
     uint32_t err = 0;
     MGX_HIP(hipMemcpyAsync(c_->h_pinned + 1, d_res_, sizeof(uint32_t), hipMemcpyDeviceToHost,
                            c_->stream));

@@ -292,6 +292,7 @@ struct Ctx {
   // (resident solves where they fit), 0 never, 1 wherever a form fits, > 1
   // CG only, on at most that many blocks
   int use_persistent = -1;
+  int64_t res_iters = 1 << 17;  // iterations of one launch of a resident solve
   // fused-engine state owned by the context (engine.hip)
   void *pool = nullptr;   // DevicePool for solver work vectors
   void *eng64 = nullptr;  // Engine<double> for single fused solves

@@ -377,6 +377,16 @@ int mgx_set_persistent(mgx_ctx *ctx, int enable) {
   });
 }
 
+// The tests' handle on resident solves (not part of the public header):
+// iterations of one launch, below 1 to make such a solve fail.
+int mgx_test_resident(mgx_ctx *ctx, int64_t iters_per_launch) {
+  return guard([&] {
+    MGX_REQUIRE(ctx, "mgx_test_resident: NULL ctx");
+    ctx->res_iters = iters_per_launch;
+    return MGX_OK;
+  });
+}
+
 // ------------------------------------------------------------- vectors ----
 int mgx_vec_create(mgx_ctx *ctx, int64_t n, mgx_dtype dtype, const void *host,
                    mgx_vec **out) {

@@ -273,24 +273,32 @@ SolveOut fused_solve(int method, Csr *A, const void *val, T *x, const T *b, int 
   cfg.rhist_len = rlen;
   int slot = eng.add(A, val, x, b, cfg);
   MGX_REQUIRE(slot >= 0, "fused solve: out of device memory for the work vectors");
-  bool done = false;
-  if (eng.resident_ok(slot) && !(done = eng.run_resident(slot))) {
-    // set the system up again for the launches
-    eng.release(slot);
-    slot = eng.add(A, val, x, b, cfg);
-    MGX_REQUIRE(slot >= 0, "fused solve: out of device memory for the work vectors");
-  }
-  if (done) {
-  } else if (eng.persistent_ok(slot)) {
-    eng.run_persistent(slot);
-  } else {
-    const int every = check_every > 0 ? check_every : 32;
-    for (;;) {
-      eng.step(every);
-      if (!eng.poll().empty()) break;
+  SolveState hs;
+  try {
+    bool done = false;
+    if (eng.resident_ok(slot) && !(done = eng.run_resident(slot))) {
+      // set the system up again for the launches
+      eng.release(slot);
+      slot = eng.add(A, val, x, b, cfg);
+      MGX_REQUIRE(slot >= 0, "fused solve: out of device memory for the work vectors");
     }
+    if (done) {
+    } else if (eng.persistent_ok(slot)) {
+      eng.run_persistent(slot);
+    } else {
+      const int every = check_every > 0 ? check_every : 32;
+      for (;;) {
+        eng.step(every);
+        if (!eng.poll().empty()) break;
+      }
+    }
+    hs = eng.state(slot);
+  } catch (...) {
+    // a slot left behind would be stepped by the context's next solve, on a
+    // matrix and vectors that may be gone by then
+    if (slot >= 0) eng.release(slot);
+    throw;
   }
-  SolveState hs = eng.state(slot);
   eng.release(slot);
   if (rlen > 0) {
     const int64_t got = std::min<int64_t>(hs.iter, rlen);

@@ -2,6 +2,7 @@
 reference's arithmetic and the oracle's tile-order dots, so FP64 and FP32 runs
 must reproduce the oracle's iterates bit for bit: same x, same iteration count,
 same residual history -- in the reference-shaped mode and in the fused mode."""
+import ctypes as C
 import os
 import sys
 
@@ -289,6 +290,36 @@ def test_resident_solves_equal_launches(m, oracle, n, reach, dtype):
                                        tol=tol, maxiter=iters, history=True)
                     assert r1.status == ref[0] and r1.final_iter == ref[2]
                     assert bits_equal(x1, ref[1])
+
+
+def resident_hook(m, ctx, iters=1 << 17):
+    """Iterations of one launch of the context's resident solves (0: such a
+    solve fails after its set-up)."""
+    m.check(m._lib.mgx_test_resident(ctx.handle, C.c_int64(iters)))
+
+
+@pytest.mark.parametrize("method", ["cg", "bicgstab"])
+def test_failed_solve_leaves_no_system_behind(m, oracle, method):
+    """A fused solve that fails after its system entered the engine: the
+    context's next solve iterates its own system only (the failed one's x
+    stays as it was), and equals the oracle's."""
+    rp, ci, val = _ring(1500, 2, 3)
+    n = len(rp) - 1
+    b = oracle.random_vector(n, -1.0, 1.0, 5)
+    tol = 1e-9 * float(oracle.nrm2(b))
+    say("failed solve", method)
+    with m.Context(0) as c:
+        A, X, B = m.CRS(c, n, n, rp, ci, val), m.Vector(c, np.full(n, 0.25)), m.Vector(c, b)
+        resident_hook(m, c, 0)
+        with pytest.raises(m.MgxError):
+            getattr(m, method)(A, X, B, tol=tol, precond=m.PRECOND_JACOBI, mode=m.MODE_FUSED)
+        resident_hook(m, c)
+        ref = oracle.solve(method, rp, ci, val, np.zeros(n), b, precond=2, tol=tol)
+        res, x = gpu_solve(m, c, method, rp, ci, val, np.zeros(n), b, m.PRECOND_JACOBI, tol,
+                           mode=m.MODE_FUSED)
+        assert res.status == ref[0] == 0 and res.final_iter == ref[2]
+        assert bits_equal(x, ref[1])
+        assert bits_equal(X.download(), np.full(n, 0.25))
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
