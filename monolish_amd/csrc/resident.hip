@@ -81,7 +81,7 @@ __global__ __launch_bounds__(kBlock) void k_res_clear(typename Slot<T>::U *slots
 template <class T> struct ResDesc {
   const int32_t *rp, *ci;
   const T *val, *M;
-  T *x, *r, *z, *pa, *pb, *r0, *va;
+  T *x, *r, *z, *pa, *pb, *r0, *va, *vb;
   double *rhist;
   int64_t rhist_len, n, ntiles;
   SolveState *st;
@@ -99,6 +99,7 @@ template <class T> struct ResDesc {
     pb = (decltype(pb))c->pb.p;
     r0 = (decltype(r0))c->r0.p;
     va = (decltype(va))c->va.p;
+    vb = (decltype(vb))c->vb.p;
     rhist = (decltype(rhist))c->rhist.p;
     st = (SolveState *)c->st.p;
     rhist_len = c->rhist_len, n = c->n, ntiles = c->ntiles;
@@ -417,7 +418,10 @@ __global__ __launch_bounds__(kBlock *TT) void k_resident_cg(const SysDesc<T> *sy
 }
 
 // BiCGSTAB (bicgstab.cpp:53-129) as k_bcg_p ... k_bcg_update compute it; three
-// all-to-all steps and two gathers (r, v) an iteration
+// all-to-all steps and two gathers (r, v) an iteration.  From one launch to
+// the next p and v go through pa and vb, which are only written at a launch's
+// end: va is written before the first step, when another block may not have
+// taken the last launch's values yet
 template <class T, int TT, int TR, int KE>
 __global__ __launch_bounds__(kBlock *TT) void k_resident_bcg(const SysDesc<T> *sys,
                                                              typename Slot<T>::U *slots,
@@ -447,7 +451,7 @@ __global__ __launch_bounds__(kBlock *TT) void k_resident_bcg(const SysDesc<T> *s
       r[k][e] = R.load(d.r, k, e);
       r0[k][e] = R.load(d.r0, k, e);
       p[k][e] = first ? T(0) : R.load(d.pa, k, e);
-      v[k][e] = first ? T(0) : R.load(d.va, k, e);
+      v[k][e] = first ? T(0) : R.load(d.vb, k, e);
       m[k][e] = d.M ? R.load(d.M, k, e) : T(1);
     }
   int32_t s = kStatRunning;
@@ -455,7 +459,7 @@ __global__ __launch_bounds__(kBlock *TT) void k_resident_bcg(const SysDesc<T> *s
   T gp[TR][2][KE], gv[TR][2][KE], gr[TR][2][KE], gm[TR][2][KE], gh[TR][2][KE];
   if (!first) {
     R.gather(d.pa, gp);
-    R.gather(d.va, gv);
+    R.gather(d.vb, gv);
   }
   if (d.M) R.gather(d.M, gm);
   while (it < stop_at) {
@@ -579,6 +583,7 @@ __global__ __launch_bounds__(kBlock *TT) void k_resident_bcg(const SysDesc<T> *s
         const int64_t i = R.row[k] + e;
         d.x[i] = x[k][e];
         d.pa[i] = p[k][e];
+        d.vb[i] = v[k][e];
       }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->beta = (double)beta;

@@ -323,6 +323,34 @@ def test_failed_solve_leaves_no_system_behind(m, oracle, method):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,reach", [(700, 2), (60001, 3), (131073, 2), (262145, 2)])
+@pytest.mark.parametrize("method", ["cg", "bicgstab"])
+def test_resident_solve_in_several_launches(m, oracle, method, n, reach, dtype):
+    """A resident solve in launches of 1 to 5 iterations each (the state goes
+    through memory between them, both parities of p): x, iterations, residual
+    and history are the launch-per-stage form's bits, for one right-hand side
+    after another."""
+    if method == "bicgstab" and n > 262144:
+        pytest.skip("not a resident size")
+    rp, ci, val = _ring(n, reach, n)
+    val = val.astype(dtype)
+    say("resident launches", method, n, dtype.__name__)
+    with m.Context(0) as own, m.Context(0) as staged:
+        m.set_persistent(staged, False)
+        for k, iters in enumerate((3, 1, 2, 5)):
+            b = oracle.random_vector(n, -1.0, 1.0, 50 + k, dtype=dtype)
+            x0 = oracle.random_vector(n, -1.0, 1.0, 60 + k, dtype=dtype)
+            tol = float((1e-9 if dtype == np.float64 else 1e-4) * oracle.nrm2(b))
+            resident_hook(m, own, iters)
+            (r1, x1), (r2, x2) = [gpu_solve(m, c, method, rp, ci, val, x0, b, m.PRECOND_JACOBI,
+                                            tol, maxiter=12, mode=m.MODE_FUSED, history=12)
+                                  for c in (own, staged)]
+            assert (r1.status, r1.final_iter) == (r2.status, r2.final_iter), iters
+            assert bits_equal(x1, x2) and bits_equal(r1.rhistory, r2.rhistory), iters
+            assert r1.final_resid == r2.final_resid, iters
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_cg_fused_large_split_iteration(m, ctx, oracle, dtype):
     """n >= 2^19 rows: the fused solver runs the split iteration (p update,
     plan-based SpMV, <p, q>, update); 40 iterations stay bit-identical to the
