@@ -149,11 +149,14 @@ void batch_launch_cg_persist(Ctx *c, const SysDesc<T> *sys, GridSync *gs, int gr
 bool resident_fits(const Ctx *c, const Csr *A, int method);
 size_t resident_bytes(int64_t ntiles);  // scratch of a launch
 // up to max_iters iterations of the single system sys[0] (CG or BiCGSTAB);
-// the first word of scratch is nonzero afterwards when a wait gave up: x
-// and the solve state are then as they were
+// the first word of scratch is nonzero afterwards when a wait gave up: x and
+// the solve state are then of no use (a block may give up at a step that
+// others pass).  keep (or nullptr) takes a copy of x, rows entries, before
+// the launch
 template <class T>
 void resident_launch(Ctx *c, int method, const SysDesc<T> *sys, int64_t ntiles, int max_row,
-                     void *scratch, int32_t *stopped, int64_t max_iters);
+                     void *scratch, int32_t *stopped, int64_t max_iters, const T *x, T *keep,
+                     int64_t rows);
 
 // set-up of newly admitted systems: scatter their staged descriptors and
 // states into their slots, then (over the list of their tiles) M = 1/diag,
@@ -267,8 +270,8 @@ template <class T> class Engine {
   void run_persistent(int slot);
   // the one running system fits a resident solve and the context allows it
   bool resident_ok(int slot) const;
-  // iterate it to its end that way; false when the blocks did not meet in
-  // time (x untouched, the work vectors not)
+  // iterate it to its end that way; false when the blocks of a launch did
+  // not meet in time (x is then what it was before, the work vectors not)
   bool run_resident(int slot);
 
  private:

@@ -293,6 +293,7 @@ struct Ctx {
   // CG only, on at most that many blocks
   int use_persistent = -1;
   int64_t res_iters = 1 << 17;  // iterations of one launch of a resident solve
+  int res_give_up = 0;  // tests: the launch after which the host reports a given-up wait
   // fused-engine state owned by the context (engine.hip)
   void *pool = nullptr;   // DevicePool for solver work vectors
   void *eng64 = nullptr;  // Engine<double> for single fused solves

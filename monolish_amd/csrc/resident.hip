@@ -67,12 +67,16 @@ template <class V> __device__ __forceinline__ void rput(V *p, V v) {
 __device__ __forceinline__ double rsqrt_of(double v) { return __builtin_sqrt(v); }
 __device__ __forceinline__ float rsqrt_of(float v) { return __builtin_sqrtf(v); }
 
+// before a launch; the first launch of a solve also keeps its x: when a wait
+// of a launch gives up, some blocks may have stored their rows all the same
 template <class T>
 __global__ __launch_bounds__(kBlock) void k_res_clear(typename Slot<T>::U *slots, int64_t n,
-                                                      uint32_t *err) {
+                                                      uint32_t *err, const T *x, T *keep,
+                                                      int64_t rows) {
   const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if (i < n) slots[i] = Slot<T>::kEmpty;
   if (i == 0) *err = 0u;
+  if (keep && i < rows) keep[i] = x[i];
 }
 
 // the descriptor's fields, read once by scalar loads into registers (read
@@ -635,12 +639,15 @@ size_t resident_bytes(int64_t ntiles) { return 256 + (size_t)ntiles * 6 * kCopie
 
 template <class T>
 void resident_launch(Ctx *c, int method, const SysDesc<T> *sys, int64_t ntiles, int max_row,
-                     void *scratch, int32_t *stopped, int64_t max_iters) {
+                     void *scratch, int32_t *stopped, int64_t max_iters, const T *x, T *keep,
+                     int64_t rows) {
   using U = typename Slot<T>::U;
   uint32_t *err = static_cast<uint32_t *>(scratch);
   U *slots = reinterpret_cast<U *>(static_cast<char *>(scratch) + 256);
   const int64_t n = 6 * kCopies * ntiles;
-  k_res_clear<T><<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, c->stream>>>(slots, n, err);
+  const int64_t nc = keep ? std::max(n, rows) : n;
+  k_res_clear<T><<<(unsigned)((nc + kBlock - 1) / kBlock), kBlock, 0, c->stream>>>(slots, n, err, x,
+                                                                                   keep, rows);
   const ResShape sp = res_shape(c, ntiles);
   ResKernel<T> k = max_row <= 5 ? res_kernel<T, 5>(method, sp.tt, sp.tr)
                                 : res_kernel<T, kEnt>(method, sp.tt, sp.tr);
@@ -650,8 +657,8 @@ void resident_launch(Ctx *c, int method, const SysDesc<T> *sys, int64_t ntiles, 
                                      dim3((unsigned)(kBlock * sp.tt)), args, 0, c->stream));
 }
 template void resident_launch<double>(Ctx *, int, const SysDesc<double> *, int64_t, int, void *,
-                                      int32_t *, int64_t);
+                                      int32_t *, int64_t, const double *, double *, int64_t);
 template void resident_launch<float>(Ctx *, int, const SysDesc<float> *, int64_t, int, void *,
-                                     int32_t *, int64_t);
+                                     int32_t *, int64_t, const float *, float *, int64_t);
 
 }  // namespace mgx

@@ -378,11 +378,14 @@ int mgx_set_persistent(mgx_ctx *ctx, int enable) {
 }
 
 // The tests' handle on resident solves (not part of the public header):
-// iterations of one launch, below 1 to make such a solve fail.
-int mgx_test_resident(mgx_ctx *ctx, int64_t iters_per_launch) {
+// iterations of one launch, below 1 to make such a solve fail, and the launch
+// of a solve (1, 2, ...; 0: none) after which the host takes its wait to have
+// given up, whatever the kernel did.
+int mgx_test_resident(mgx_ctx *ctx, int64_t iters_per_launch, int give_up_launch) {
   return guard([&] {
     MGX_REQUIRE(ctx, "mgx_test_resident: NULL ctx");
     ctx->res_iters = iters_per_launch;
+    ctx->res_give_up = give_up_launch;
     return MGX_OK;
   });
 }
