@@ -133,7 +133,10 @@ int mgx_set_graphs(mgx_ctx *ctx, int enable);
  * between the stages).  A value above 1: CG systems small enough for the
  * two-kernel iteration, in one cooperative launch of at most that many
  * blocks (each then owns several 128-row quarters).  The results are the
- * same bits in every form. */
+ * same bits in every form.  Where the device refuses the launch of a resident
+ * solve, or its blocks wait for each other for more than 2 s (compute units
+ * held by other work), the solve runs again one launch per stage, and so do
+ * the context's later ones until this is called again. */
 int mgx_set_persistent(mgx_ctx *ctx, int enable);
 
 /* ---- vectors: vector<T>::send/recv/nonfree_recv/device_free ------------- */

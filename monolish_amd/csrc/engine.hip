@@ -502,7 +502,8 @@ template <class T> void Engine<T>::run_persistent(int slot) {
 // launch-per-stage solves, for a capped grid or for graph replay.  Measured on
 // one system, FP64, resident against the launches: see resident.hip.
 template <class T> bool Engine<T>::resident_ok(int slot) const {
-  if (c_->use_persistent == 0 || c_->use_persistent > 1 || c_->use_graphs) return false;
+  if (c_->use_persistent == 0 || c_->use_persistent > 1 || c_->use_graphs || c_->res_off)
+    return false;
   if (active_.size() != 1 || active_[0] != slot) return false;
   return !h_sys_[slot].split && resident_fits(c_, csr_[slot], method_[slot]);
 }
@@ -515,7 +516,14 @@ template <class T> bool Engine<T>::run_resident(int slot) {
   if (bytes > res_cap_) {
     dev_free(d_res_);
     d_res_ = nullptr;
-    d_res_ = dev_alloc(bytes);
+    res_cap_ = 0;
+    try {
+      d_res_ = dev_alloc(bytes);
+    } catch (const Error &e) {
+      if (e.code != MGX_ERR_NOMEM) throw;
+      (void)hipGetLastError();
+      return false;
+    }
     res_cap_ = bytes;
   }
   // a launch ends after this many iterations (a second or two); the host
@@ -526,15 +534,22 @@ template <class T> bool Engine<T>::run_resident(int slot) {
   const SysDesc<T> &h = h_sys_[slot];
   T *const keep = method_[slot] == kMethodCG ? h.q : h.t;
   for (int launch = 1;; launch++) {
-    resident_launch<T>(c_, method_[slot], d_sys_ + slot, nt, csr_[slot]->plan.max_row, d_res_,
-                       d_stopped_, per_launch, h.x, launch == 1 ? keep : nullptr, h.n);
-    uint32_t err = 0;
-    MGX_HIP(hipMemcpyAsync(c_->h_pinned + 1, d_res_, sizeof(uint32_t), hipMemcpyDeviceToHost,
-                           c_->stream));
-    const bool stopped = !poll().empty();
-    std::memcpy(&err, c_->h_pinned + 1, sizeof err);
-    if (launch == c_->res_give_up) err = 1;  // (as the tests set it)
-    if (err != 0) {
+    bool ok = resident_launch<T>(c_, method_[slot], d_sys_ + slot, nt, csr_[slot]->plan.max_row,
+                                 d_res_, d_stopped_, per_launch, h.x,
+                                 launch == 1 ? keep : nullptr, h.n);
+    if (launch == -c_->res_give_up) ok = false;  // (as the tests set it)
+    bool stopped = false;
+    if (ok) {
+      uint32_t err = 0;
+      MGX_HIP(hipMemcpyAsync(c_->h_pinned + 1, d_res_, sizeof(uint32_t), hipMemcpyDeviceToHost,
+                             c_->stream));
+      stopped = !poll().empty();
+      std::memcpy(&err, c_->h_pinned + 1, sizeof err);
+      ok = err == 0 && launch != c_->res_give_up;
+    }
+    if (!ok) {
+      // what keeps the blocks apart may last: no more of these launches
+      c_->res_off = true;
       MGX_HIP(hipMemcpyAsync(h.x, keep, (size_t)h.n * sizeof(T), hipMemcpyDeviceToDevice,
                              c_->stream));
       return false;

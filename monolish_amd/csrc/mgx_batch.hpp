@@ -152,9 +152,10 @@ size_t resident_bytes(int64_t ntiles);  // scratch of a launch
 // the first word of scratch is nonzero afterwards when a wait gave up: x and
 // the solve state are then of no use (a block may give up at a step that
 // others pass).  keep (or nullptr) takes a copy of x, rows entries, before
-// the launch
+// the launch.  False when the runtime refuses the launch (its blocks would not
+// all be resident, as with masked compute units)
 template <class T>
-void resident_launch(Ctx *c, int method, const SysDesc<T> *sys, int64_t ntiles, int max_row,
+bool resident_launch(Ctx *c, int method, const SysDesc<T> *sys, int64_t ntiles, int max_row,
                      void *scratch, int32_t *stopped, int64_t max_iters, const T *x, T *keep,
                      int64_t rows);
 
@@ -270,8 +271,10 @@ template <class T> class Engine {
   void run_persistent(int slot);
   // the one running system fits a resident solve and the context allows it
   bool resident_ok(int slot) const;
-  // iterate it to its end that way; false when the blocks of a launch did
-  // not meet in time (x is then what it was before, the work vectors not)
+  // iterate it to its end that way; false when a launch was refused or its
+  // blocks did not meet in time, which the context remembers, and when there
+  // is no memory for the scratch (x is then what it was before, the work
+  // vectors are not)
   bool run_resident(int slot);
 
  private:

@@ -294,6 +294,8 @@ struct Ctx {
   int use_persistent = -1;
   int64_t res_iters = 1 << 17;  // iterations of one launch of a resident solve
   int res_give_up = 0;  // tests: the launch after which the host reports a given-up wait
+                        // (negative: the launch that it takes to be refused)
+  bool res_off = false;  // a resident launch was refused or gave up (until mgx_set_persistent)
   // fused-engine state owned by the context (engine.hip)
   void *pool = nullptr;   // DevicePool for solver work vectors
   void *eng64 = nullptr;  // Engine<double> for single fused solves

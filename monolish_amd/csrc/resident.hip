@@ -638,7 +638,7 @@ bool resident_fits(const Ctx *c, const Csr *A, int method) {
 size_t resident_bytes(int64_t ntiles) { return 256 + (size_t)ntiles * 6 * kCopies * 8; }
 
 template <class T>
-void resident_launch(Ctx *c, int method, const SysDesc<T> *sys, int64_t ntiles, int max_row,
+bool resident_launch(Ctx *c, int method, const SysDesc<T> *sys, int64_t ntiles, int max_row,
                      void *scratch, int32_t *stopped, int64_t max_iters, const T *x, T *keep,
                      int64_t rows) {
   using U = typename Slot<T>::U;
@@ -653,12 +653,17 @@ void resident_launch(Ctx *c, int method, const SysDesc<T> *sys, int64_t ntiles, 
                                 : res_kernel<T, kEnt>(method, sp.tt, sp.tr);
   void *args[] = {(void *)&sys, (void *)&slots, (void *)&err, (void *)&stopped,
                   (void *)&max_iters};
-  MGX_HIP(hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3((unsigned)sp.grid),
-                                     dim3((unsigned)(kBlock * sp.tt)), args, 0, c->stream));
+  MGX_HIP(hipGetLastError());
+  const hipError_t e =
+      hipLaunchCooperativeKernel(reinterpret_cast<const void *>(k), dim3((unsigned)sp.grid),
+                                 dim3((unsigned)(kBlock * sp.tt)), args, 0, c->stream);
+  if (e == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
 }
-template void resident_launch<double>(Ctx *, int, const SysDesc<double> *, int64_t, int, void *,
+template bool resident_launch<double>(Ctx *, int, const SysDesc<double> *, int64_t, int, void *,
                                       int32_t *, int64_t, const double *, double *, int64_t);
-template void resident_launch<float>(Ctx *, int, const SysDesc<float> *, int64_t, int, void *,
+template bool resident_launch<float>(Ctx *, int, const SysDesc<float> *, int64_t, int, void *,
                                      int32_t *, int64_t, const float *, float *, int64_t);
 
 }  // namespace mgx

@@ -373,6 +373,7 @@ int mgx_set_persistent(mgx_ctx *ctx, int enable) {
     MGX_REQUIRE(ctx, "mgx_set_persistent: NULL ctx");
     MGX_REQUIRE(enable >= 0, "mgx_set_persistent: negative value");
     ctx->use_persistent = enable;
+    ctx->res_off = false;
     return MGX_OK;
   });
 }
@@ -380,7 +381,8 @@ int mgx_set_persistent(mgx_ctx *ctx, int enable) {
 // The tests' handle on resident solves (not part of the public header):
 // iterations of one launch, below 1 to make such a solve fail, and the launch
 // of a solve (1, 2, ...; 0: none) after which the host takes its wait to have
-// given up, whatever the kernel did.
+// given up, whatever the kernel did; -1, -2, ...: the launch that it takes to
+// have been refused.
 int mgx_test_resident(mgx_ctx *ctx, int64_t iters_per_launch, int give_up_launch) {
   return guard([&] {
     MGX_REQUIRE(ctx, "mgx_test_resident: NULL ctx");

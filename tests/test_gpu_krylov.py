@@ -295,7 +295,7 @@ def test_resident_solves_equal_launches(m, oracle, n, reach, dtype):
 def resident_hook(m, ctx, iters=1 << 17, give_up=0):
     """Iterations of one launch of the context's resident solves (0: such a
     solve fails after its set-up), and the launch after which the host takes
-    its wait to have given up (0: none)."""
+    its wait to have given up (0: none; -k: launch k taken to be refused)."""
     m.check(m._lib.mgx_test_resident(ctx.handle, C.c_int64(iters), C.c_int(give_up)))
 
 
@@ -351,14 +351,16 @@ def test_resident_solve_in_several_launches(m, oracle, method, n, reach, dtype):
             assert r1.final_resid == r2.final_resid, iters
 
 
-@pytest.mark.parametrize("iters,give_up", [(1 << 17, 1), (2, 1), (2, 2), (1, 3)])
+@pytest.mark.parametrize("iters,give_up", [(1 << 17, 1), (2, 1), (2, 2), (1, 3), (1 << 17, -1),
+                                           (2, -2)])
 @pytest.mark.parametrize("n", [700, 200001])
 @pytest.mark.parametrize("method", ["cg", "bicgstab"])
 def test_resident_wait_that_gave_up(m, oracle, method, n, iters, give_up):
     """A wait that gave up (here: the host says so, after a launch that wrote
-    all of x), in the only launch of a solve, its first or a later one: the
-    solve runs again in launches per stage from the caller's x, with their
-    bits, iterations and history."""
+    all of x), in the only launch of a solve, its first or a later one, and a
+    launch that was refused: the solve runs again in launches per stage from
+    the caller's x, with their bits, iterations and history, and so does the
+    context's next one (a resident one would fail here)."""
     rp, ci, val = _ring(n, 2, n)
     b = oracle.random_vector(n, -1.0, 1.0, 5)
     x0 = oracle.random_vector(n, -1.0, 1.0, 6)
@@ -373,6 +375,14 @@ def test_resident_wait_that_gave_up(m, oracle, method, n, iters, give_up):
         assert r1.status == r2.status and r1.final_iter == r2.final_iter > 3
         assert bits_equal(x1, x2) and bits_equal(r1.rhistory, r2.rhistory)
         assert r1.final_resid == r2.final_resid
+        resident_hook(m, own, 0)  # no iterations: a resident solve raises
+        r1, x1 = gpu_solve(m, own, method, rp, ci, val, x0, b, m.PRECOND_JACOBI, tol,
+                           maxiter=12, mode=m.MODE_FUSED)
+        assert r1.final_iter == r2.final_iter and bits_equal(x1, x2)
+        m.set_persistent(own, True)  # asks for them again
+        with pytest.raises(m.MgxError):
+            gpu_solve(m, own, method, rp, ci, val, x0, b, m.PRECOND_JACOBI, tol, maxiter=12,
+                      mode=m.MODE_FUSED)
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
