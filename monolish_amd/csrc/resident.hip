@@ -47,6 +47,7 @@ constexpr int kResLanes = 4;      // partials per stage-2 lane: 1024 tiles
 // copies of every partial, one for the blocks of each XCD
 constexpr int kCopies = 8;
 constexpr uint64_t kResTicks = 200000000;  // 2 s of the 100 MHz clock
+constexpr uint64_t kResGap = 1000000;      // 10 ms, what 1024 reads never take
 
 template <class T> struct Slot;
 template <> struct Slot<double> {
@@ -192,7 +193,7 @@ template <class T, int TT, int TR, int KE> struct Resident {
   // added); res[v] for every thread; false when a wait gave up
   template <int NV>
   __device__ __forceinline__ bool meet(const T (&a)[NV][TR], T (&res)[NV]) {
-        const int lane = threadIdx.x & 63, wv = threadIdx.x / 64, g = threadIdx.x / kBlock;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x / 64, g = threadIdx.x / kBlock;
     const int64_t nt = d.ntiles;
     U *const set = slots + (int64_t)(step % 3) * kCopies * 2 * nt;
     U *const prev = slots + (int64_t)((step + 2) % 3) * kCopies * 2 * nt;
@@ -234,7 +235,8 @@ template <class T, int TT, int TR, int KE> struct Resident {
       for (int j = 0; j < kResLanes; j++)
 #pragma unroll
         for (int v = 0; v < NV; v++) got[v][j] = Slot<T>::kEmpty;
-      uint64_t t0 = 0;
+      uint64_t last = 0, waited = 0;
+      bool late = false;  // out of time: one more read decides
       for (uint32_t spin = 0;; spin++) {
         // only what is missing is asked for again
         bool miss = false;
@@ -253,14 +255,18 @@ template <class T, int TT, int TR, int KE> struct Resident {
             for (int v = 0; v < NV; v++) miss = miss || got[v][j] == Slot<T>::kEmpty;
           }
         if (!__any(miss)) break;
+        if (late) {
+          rput(err, 1u);
+          ok = 0;
+          break;
+        }
         if ((spin & 1023u) == 1023u) {
+          // (a longer gap between two looks: all blocks stood still, the
+          // process was taken off the device)
           const uint64_t now = wall_clock64();
-          if (t0 == 0) t0 = now;
-          if (now - t0 > kResTicks || rget(err) != 0u) {
-            rput(err, 1u);
-            ok = 0;
-            break;
-          }
+          if (last) waited += min(now - last, kResGap);
+          last = now;
+          late = waited > kResTicks || rget(err) != 0u;
         }
       }
 #pragma unroll
@@ -635,6 +641,7 @@ bool resident_fits(const Ctx *c, const Csr *A, int method) {
          (method == kMethodCG || sp.tr == 1);
 }
 
+// (the slots of FP64 sums; FP32 ones take half)
 size_t resident_bytes(int64_t ntiles) { return 256 + (size_t)ntiles * 6 * kCopies * 8; }
 
 template <class T>
