@@ -479,17 +479,19 @@ __global__ __launch_bounds__(kBlock) void k_spmv_pat(
   const int nth = (int)blockDim.x, t = (int)threadIdx.x;
   const int64_t r0 = b * nth, r = r0 + t, rc = r < rows ? r : rows - 1;
   const int32_t e0 = rp[r0], e1 = rp[r0 + nth < rows ? r0 + nth : rows];
-  const int32_t ea = e0 & ~(W - 1);
+  const int32_t ea = e0 & ~(W - 1), ne = e1 - ea;
   const int32_t id = pt.id[rc], ra = rp[rc];
-  for (int32_t k0 = ea + t * W; k0 < e1; k0 += G * nth * W) {
+  // counted from ea: positions beyond e1 may not fit 32 bits
+  const T *const bv = val + ea;
+  for (int32_t k0 = t * W; k0 < ne; k0 += G * nth * W) {
     VT v[G];
 #pragma unroll
     for (int k = 0; k < G; k++)
-      if (k0 + k * nth * W < e1)
-        v[k] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(val + k0 + k * nth * W));
+      if (k0 + k * nth * W < ne)
+        v[k] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(bv + k0 + k * nth * W));
 #pragma unroll
     for (int k = 0; k < G; k++)
-      if (k0 + k * nth * W < e1) *reinterpret_cast<VT *>(sv + (k0 - ea) + k * nth * W) = v[k];
+      if (k0 + k * nth * W < ne) *reinterpret_cast<VT *>(sv + k0 + k * nth * W) = v[k];
   }
   sell_pat_stage(pt, pat_lds);
   __syncthreads();

@@ -677,6 +677,40 @@ def test_sliced_row_patterns(m, ctx, oracle, dtype, rows, npat, lens, span):
         o.free()
 
 
+def test_entry_positions_next_to_2_31(m, ctx):
+    """The largest entry count that fits 32-bit row pointers: positions just
+    past a block's last entry don't, so no block may form them.  Rows of 24
+    consecutive columns (one row pattern) and exact small-integer sums, so
+    that y is known without a second product."""
+    have = os.sysconf("SC_AVPHYS_PAGES") * os.sysconf("SC_PAGE_SIZE")
+    if have < 64 << 30:
+        pytest.skip("needs 64 GB of free host memory")
+    L = 24
+    rows = (2**31 - 2) // L
+    nnz = rows * L
+    assert 2**31 - 2 - nnz < 64
+    say("2^31 entries", nnz)
+    ci = (np.arange(rows, dtype=np.int32)[:, None] + np.arange(L, dtype=np.int32)).reshape(-1)
+    say("columns made")
+    rp = np.arange(0, nnz + 1, L, dtype=np.int32)
+    A = m.CRS(ctx, rows, rows + L, rp, ci, np.ones(nnz, np.float32))
+    del ci
+    say("uploaded")
+    x = (np.arange(rows + L) % 13).astype(np.float32)
+    X, Y = m.Vector(ctx, x, dtype=np.float32), m.Vector(ctx, n=rows, dtype=np.float32)
+    c = np.concatenate([[0], np.cumsum(x.astype(np.int64))])
+    ref = (c[L:L + rows] - c[:rows]).astype(np.float32)
+    for plan in (None,):
+        if plan:
+            A.set_plan(**plan)
+        Y.fill(-1.0)
+        m.matvec(A, X, Y)
+        assert np.array_equal(Y.download(), ref), plan
+        say("plan done", plan)
+    for o in (A, X, Y):
+        o.free()
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_dot_nrm2_device_results(m, ctx, oracle, dtype):
     """mgx_dot_device / mgx_nrm2_device leave the result in device memory:
