@@ -72,7 +72,7 @@ def streamed_bytes(plan, nnz: int, rows: int, cols: int, sv: int, patterns: bool
     """What the plan's kernel cannot do without: the CRS arrays, or, where
     row patterns stand in for the columns, a byte per row instead (and the
     slice offsets, or row_ptr in the block plan)."""
-    if not patterns or plan["column_panels"] or plan["row_walk"] not in (0, 2):
+    if plan["row_walk"] != 4 and not (patterns and plan["row_walk"] == 2):
         return spmv_bytes(nnz, rows, cols, sv)
     meta = rows // 4 if plan["row_walk"] == 2 else (rows + 1) * 4
     return nnz * sv + rows + meta + cols * sv + rows * sv
@@ -794,7 +794,7 @@ def spmv_kernel_name(plan, dtype, patterns=False) -> str:
         return f"k_spmv_sell<{t}, false, {w}, {'true' if patterns else 'false'}>"
     if plan["column_panels"]:
         return f"k_spmv_panel<{t}"
-    if patterns and plan["row_walk"] == 0:
+    if plan["row_walk"] == 4:
         return f"k_spmv_pat<{t}, false>"
     u = (plan["nnz_per_block"] + w - 1 + 256 * w - 1) // (256 * w)
     u = next(k for k in (1, 2, 3, 4, 5, 6, 8, 9, 12, 17) if u <= k)
@@ -845,7 +845,7 @@ def main():
     ap.add_argument("--plan", default="",
                     help="fix the headline SpMV plan instead of autotuning: "
                          "'row_walk,rows_per_block,nnz_per_block,xcd_remap,column_panels' "
-                         "(row_walk 2 = sliced layout); for profiling runs")
+                         "(row_walk 2 = sliced layout, 4 = row patterns); for profiling runs")
     ap.add_argument("--traffic-probe", default="",
                     help="c2a|c2b[:f32]: only run 5 vadd launches of known size (counter "
                          "calibration), then 5 SpMVs on that matrix under --plan (else the "

@@ -69,7 +69,10 @@ int mgx_set_stream(mgx_ctx *ctx, void *stream);
 int mgx_device_info(mgx_ctx *ctx, char *name, size_t len, int *compute_units,
                     size_t *hbm_bytes);
 /* SpMV tuning: rows per block limit, entries per block limit, long-row
- * threshold, XCD-aware block order.  Applies to CRS created afterwards. */
+ * threshold, XCD-aware block order.  Applies to CRS created afterwards, which
+ * then start with exactly that block plan (until the call, a large matrix
+ * whose rows hold few distinct lists of column - row starts with row_walk 4,
+ * see mgx_spmv_tuning). */
 int mgx_set_spmv_tuning(mgx_ctx *ctx, int rows_per_block, int nnz_per_block,
                         int long_row, int xcd_remap);
 /* Autotuner of the SpMV block plan (no monolish counterpart: monolish hands
@@ -84,7 +87,8 @@ int mgx_set_spmv_tuning(mgx_ctx *ctx, int rows_per_block, int nnz_per_block,
  * entries by at most 30 %, the sliced layout (entries stored a second time
  * in 64-row slices of 16-byte tuples, one lane per row, no LDS) in launch
  * order, with one range of row blocks per XCD, and with runs of 16 row
- * blocks dealt to the XCDs in turn -- `reps` launches each; keeps the
+ * blocks dealt to the XCDs in turn, and row patterns in the same three
+ * orders where the matrix has them -- `reps` launches each; keeps the
  * fastest for A and reports it
  * (within 2 %, an XCD-ordered block plan).  The long-row threshold is
  * unchanged, so results do not depend on the choice.  The column-panel and
@@ -95,15 +99,16 @@ typedef struct mgx_spmv_tuning {
   double us;           /* time of one SpMV under the chosen plan */
   int32_t candidates;  /* plans timed */
   int32_t column_panels; /* 0, or the column panels of the chosen plan */
-  int32_t row_walk;    /* 0 products staged in LDS in entry order (a large
-                          matrix whose rows hold few distinct lists of
-                          column - row: values staged, a lane per row, in
-                          blocks of the library's choice); 1 row
+  int32_t row_walk;    /* 0 products staged in LDS in entry order; 1 row
                           walk (lane per row over LDS-staged val / col_ind;
                           coalesced gathers on banded rows); 2 the sliced
                           layout; 3 L2 panels (row sums kept in LDS while the
                           blocks walk column panels of about 0.5-2 MiB of x,
-                          column_panels of them) */
+                          column_panels of them); 4 row patterns (a matrix
+                          whose rows hold few distinct lists of column - row:
+                          values staged, a lane per row, columns from a
+                          table, in blocks of 256 or 128 rows whatever
+                          rows_per_block and nnz_per_block say) */
   int32_t pad;
 } mgx_spmv_tuning;
 int mgx_csr_autotune(mgx_csr *A, int reps, mgx_spmv_tuning *out);
@@ -113,10 +118,11 @@ int mgx_csr_autotune(mgx_csr *A, int reps, mgx_spmv_tuning *out);
  * or a run length in [2, 1024] (runs of that many consecutive blocks dealt
  * to the XCDs in turn), row_walk 0/1 (block kind), 2 (the sliced
  * layout, over a product-staged block plan kept for other values; refused
- * when its padding exceeds 30 %) or 3 (L2 panels: column_panels in
- * [1, 65536], at most 2^20 columns each, ascending columns within rows),
- * column_panels 0 or 2..64 otherwise (needs ascending columns within rows;
- * not with row_walk 2): MGX_ERR_INVALID otherwise.
+ * when its padding exceeds 30 %), 3 (L2 panels: column_panels in
+ * [1, 65536], at most 2^20 columns each, ascending columns within rows) or 4
+ * (row patterns, refused where the matrix has none), column_panels 0 or 2..64
+ * otherwise (needs ascending columns within rows; not with row_walk 2 or 4):
+ * MGX_ERR_INVALID otherwise.
  * The long-row threshold stays as it is. */
 int mgx_csr_set_plan(mgx_csr *A, int rows_per_block, int nnz_per_block, int xcd_remap,
                      int row_walk, int column_panels);

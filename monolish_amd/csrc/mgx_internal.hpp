@@ -287,6 +287,7 @@ struct Ctx {
   hipEvent_t ev = nullptr;
   // SpMV tuning
   int spmv_rows = 256, spmv_nnz = 2048, spmv_long = 256, xcd_remap = 1;
+  bool spmv_fixed = false;  // the program chose them: block plans as it says
   int use_graphs = 0;  // replay fused iterations from a captured hipGraph
   // single small solves in one cooperative launch: -1 the library's choice
   // (resident solves where they fit), 0 never, 1 wherever a form fits, > 1

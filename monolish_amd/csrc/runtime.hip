@@ -304,6 +304,7 @@ int mgx_set_spmv_tuning(mgx_ctx *ctx, int rows_per_block, int nnz_per_block,
     ctx->spmv_nnz = nnz_per_block;
     ctx->spmv_long = long_row;
     ctx->xcd_remap = xcd_remap ? 1 : 0;
+    ctx->spmv_fixed = true;
     return MGX_OK;
   });
 }
@@ -333,7 +334,7 @@ int mgx_csr_set_plan(mgx_csr *A, int rows_per_block, int nnz_per_block, int xcd_
     MGX_REQUIRE(A, "mgx_csr_set_plan: NULL matrix");
     MGX_REQUIRE(rows_per_block >= 1 && rows_per_block <= kBlock,
                 "rows_per_block must be in [1, %d]", kBlock);
-    MGX_REQUIRE(row_walk >= 0 && row_walk <= 3, "row_walk must be 0, 1, 2 or 3");
+    MGX_REQUIRE(row_walk >= 0 && row_walk <= 4, "row_walk must be 0, 1, 2, 3 or 4");
     MGX_REQUIRE(xcd_remap >= 0 && xcd_remap <= kMaxRemapRun,
                 "xcd_remap must be 0, 1 or a run length in [2, %d]", kMaxRemapRun);
     // the row walk stages 12 bytes per FP64 entry in LDS: 4096 entries fit 64 KiB
@@ -349,11 +350,15 @@ int mgx_csr_set_plan(mgx_csr *A, int rows_per_block, int nnz_per_block, int xcd_
     const int long_t = A->plan.long_row > 0 ? A->plan.long_row : A->ctx->spmv_long;
     MGX_REQUIRE(long_t <= nnz_per_block, "nnz_per_block below the long-row threshold %d",
                 long_t);
-    MGX_REQUIRE(row_walk != 2 || column_panels == 0,
-                "mgx_csr_set_plan: the sliced layout and column panels exclude each other");
+    MGX_REQUIRE((row_walk != 2 && row_walk != 4) || column_panels == 0,
+                "mgx_csr_set_plan: column panels exclude the sliced layout and row patterns");
     spmv_plan_build_with(A, rp.data(), rows_per_block, nnz_per_block, long_t, xcd_remap,
                          row_walk == 1);
-    if (row_walk == 0 && !column_panels) A->plan.rowpat = spmv_rowpat_ok(A);
+    if (row_walk == 4) {
+      MGX_REQUIRE(spmv_rowpat_ok(A),
+                  "mgx_csr_set_plan: the matrix has no row patterns, or they don't fit a block");
+      A->plan.rowpat = 1;
+    }
     if (row_walk == 3)
       MGX_REQUIRE(spmv_lpanel_build(A, column_panels),
                   "mgx_csr_set_plan: L2 panels need ascending columns within rows and at "

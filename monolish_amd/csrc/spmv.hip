@@ -732,7 +732,7 @@ bool spmv_rowpat_ok(const Csr *A) {
 
 void spmv_plan_build(Ctx *c, Csr *A, const int32_t *rp) {
   spmv_plan_build_with(A, rp, c->spmv_rows, c->spmv_nnz, c->spmv_long, c->xcd_remap, 0);
-  A->plan.rowpat = spmv_rowpat_ok(A);
+  A->plan.rowpat = !c->spmv_fixed && spmv_rowpat_ok(A);
 }
 
 void spmv_plan_build_with(Csr *A, const int32_t *rp, int rows_req, int nnz_req, int long_req,
@@ -1722,7 +1722,6 @@ void spmv_autotune(Csr *A, int reps, mgx_spmv_tuning *out) {
           best_us = pat_us;
           spmv_sell_free(A);
           best_sell = 0;
-          best.walk = 0;
           A->plan.rowpat = 1;
           A->plan.remap = pat_remap;
         }
@@ -1750,7 +1749,7 @@ void spmv_autotune(Csr *A, int reps, mgx_spmv_tuning *out) {
     out->us = best_us;
     out->candidates = (int32_t)ncand;
     out->column_panels = lpanel_best ? lpanel_best : best_panels;
-    out->row_walk = best_sell ? 2 : (lpanel_best ? 3 : best.walk);
+    out->row_walk = best_sell ? 2 : lpanel_best ? 3 : A->plan.rowpat ? 4 : best.walk;
   }
 }
 

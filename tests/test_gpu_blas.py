@@ -677,6 +677,52 @@ def test_sliced_row_patterns(m, ctx, oracle, dtype, rows, npat, lens, span):
         o.free()
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_block_plans_of_a_matrix_with_row_patterns(m, oracle, dtype):
+    """Block plans that the program chooses, on a matrix that starts with row
+    patterns: the products-staged kernel in blocks of any size, the pattern
+    kernel in each order, a context with a tuning of its own, and the
+    autotuner's plan given back to set_plan; the same bits from all.  Row
+    patterns are refused where there are none."""
+    say("plans with patterns", dtype.__name__)
+    rp, ci, val = m.stencil3d(67, 59, 71, 7, 0.25)
+    val = val.astype(dtype)
+    n = len(rp) - 1
+    x = oracle.random_vector(n, -1.0, 1.0, 40, dtype=dtype)
+    ref = oracle.spmv(rp, ci, val, x)
+    with m.Context(0) as c:
+        X, Y = m.Vector(c, x, dtype=dtype), m.Vector(c, n=n, dtype=dtype)
+        A = m.CRS(c, n, n, rp, ci, val)
+
+        def same(what):
+            Y.fill(7.0)
+            m.matvec(A, X, Y)
+            assert bits_equal(Y.download(), ref), what
+
+        for plan in (dict(rows_per_block=7, nnz_per_block=512), dict(rows_per_block=256),
+                     dict(rows_per_block=64, nnz_per_block=8192, xcd_remap=0),
+                     dict(row_walk=4), dict(row_walk=4, xcd_remap=0),
+                     dict(row_walk=4, rows_per_block=1, xcd_remap=16)):
+            A.set_plan(**plan)
+            same(plan)
+        t = A.autotune(reps=2)
+        A.set_plan(**{k: t[k] for k in ("rows_per_block", "nnz_per_block", "xcd_remap", "row_walk",
+                                        "column_panels")})
+        same(t)
+        with pytest.raises(m.MgxError):
+            A.set_plan(row_walk=4, column_panels=4)
+        A.free()
+        c.set_spmv_tuning(rows_per_block=16, nnz_per_block=256, long_row=64)
+        A = m.CRS(c, n, n, rp, ci, val)
+        same("tuned context")
+        assert A.stats()["stream_blocks"] >= n // 16
+        A.free()
+        A = m.CRS(c, n - 1, n, np.minimum(rp[:-1], 200), ci[:200], val[:200])
+        with pytest.raises(m.MgxError):
+            A.set_plan(row_walk=4)
+        A.free()
+
+
 def test_entry_positions_next_to_2_31(m, ctx):
     """The largest entry count that fits 32-bit row pointers: positions just
     past a block's last entry don't, so no block may form them.  Rows of 24
