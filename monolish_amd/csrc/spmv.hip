@@ -709,21 +709,29 @@ static SellPat sell_pat(const Csr *A) {
 }
 static size_t pat_bytes(const SellPat &pt) { return (size_t)pt.n * pt.stride * 4; }
 
-// LDS of a k_spmv_pat block of `rows` rows, values of es bytes
+// LDS of a k_spmv_pat block of `rows` rows (kBlock or half of it), values of
+// es bytes: room for the block with the most entries
 static size_t rowpat_bytes(const Csr *A, int rows, size_t es) {
-  return pat_bytes(sell_pat(A)) + ((size_t)rows * A->plan.max_row + 32 / es) * es;
+  return pat_bytes(sell_pat(A)) + ((size_t)A->plan.block_ent[rows == kBlock] + 32 / es) * es;
 }
 
 // rows of a k_spmv_pat block: kBlock, or half of that where it would take more
 // than 32 KB of LDS and leave a compute unit few wavefronts (27-point 128^3
 // FP64, 59 KB: 118 us with 256 rows, 112 with 128; 16 entries a row, 33 KB:
-// 31.5 / 30.2; 27-point FP32, 31 KB: 52 / 58); 0: not even that fits, or the
-// lanes' rows start in the same bank (rows of 32 entries, FP64: products
-// staged 94.7, this 100.3)
+// 31.5 / 30.2; 27-point FP32, 31 KB: 52 / 58); 0: not even that fits, or most
+// rows start in the same bank (rows of 32 entries, FP64: products staged 94.7,
+// this 100.3), or rows of uneven length leave most of that LDS empty: where
+// LDS limits the blocks of a compute unit, they have to keep 32 KB of values
+// in flight (runs of 1000 rows of 48 entries among rows of 3, 18 KB: products
+// staged 16.2, this 28.2 us in FP64, 13.9 / 15.3 in FP32)
 static int rowpat_rows(const Csr *A, size_t es) {
-  if (A->plan.max_row % 32 == 0) return 0;
-  if (rowpat_bytes(A, kBlock, es) <= 32768) return kBlock;
-  return rowpat_bytes(A, kBlock / 2, es) <= 65536 ? kBlock / 2 : 0;
+  if (2 * A->plan.rows32 > A->rows) return 0;
+  for (int rb : {kBlock, kBlock / 2}) {
+    const size_t lds = rowpat_bytes(A, rb, es), fit = ((size_t)160 << 10) / lds;
+    if (lds > (rb == kBlock ? 32768u : 65536u)) continue;
+    if (fit * rb >= 2048 || (double)(fit * rb * es) * A->plan.mean_row >= 32768) return rb;
+  }
+  return 0;
 }
 
 bool spmv_rowpat_ok(const Csr *A) {
@@ -773,6 +781,18 @@ void spmv_plan_build_with(Csr *A, const int32_t *rp, int rows_req, int nnz_req, 
   }
   const int64_t nb = (int64_t)blk.size();
   blk.push_back(make_int2((int32_t)rows, rp[rows]));
+  A->plan.rows32 = 0;
+  for (int64_t i = 0; i < rows; i++) {
+    const int32_t len = rp[i + 1] - rp[i];
+    A->plan.rows32 += len > 0 && len % 32 == 0;
+  }
+  for (int k = 0; k < 2; k++) {
+    const int64_t step = k ? kBlock : kBlock / 2;
+    int32_t most = 0;
+    for (int64_t i = 0; i < rows; i += step)
+      most = std::max(most, rp[std::min(i + step, rows)] - rp[i]);
+    A->plan.block_ent[k] = most;
+  }
   A->plan.nblocks = nb;
   A->plan.nlong = nlong;
   A->plan.max_row = mx;
@@ -1396,9 +1416,9 @@ static void spmv_dispatch(Csr *A, const T *V, const T *X, T *Y, T alpha,
     spmv_panels_dispatch<T>(A, X, Y);
     return;
   }
-  if (A->plan.rowpat) {
+  // (an FP32 copy of the values may not qualify where the FP64 ones do)
+  if (const int rb = A->plan.rowpat ? rowpat_rows(A, sizeof(T)) : 0) {
     const SellPat pt = sell_pat(A);
-    const int rb = rowpat_rows(A, sizeof(T));
     const int64_t nb = (A->rows + rb - 1) / rb;
     const RemapGrid rg = remap_grid(A->plan.remap, nb);
     const size_t lds = rowpat_bytes(A, rb, sizeof(T));

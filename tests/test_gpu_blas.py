@@ -635,7 +635,7 @@ def pattern_rows(rng, rows, npat, lens, span):
     (100001, 2, (16, 16), 40),       # FP64: 32 KB of LDS are not enough for 256 rows
     (100127, 2, (15, 14), 40),       # and are for these
     (100129, 3, (63, 62, 61), 90),   # FP64: 128 rows take just under 64 KB
-    (100130, 3, (64, 63, 62), 90),   # and just over
+    (100130, 3, (65, 64, 63), 90),   # and just over
     (60001, 4, (32, 31, 30), 90),    # rows 32 apart in LDS: columns from memory
 ])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
@@ -674,6 +674,55 @@ def test_sliced_row_patterns(m, ctx, oracle, dtype, rows, npat, lens, span):
         assert bits_equal(Y.download(), oracle.spmv(rp, ci, v2, x)), plan
         A.free()
     for o in (X, Y):
+        o.free()
+
+
+def _uneven(kind):
+    """Rows that start at their own column: one long row in an otherwise even
+    matrix (first, last or inside), runs of long rows among short ones, a
+    ragged last block with empty rows."""
+    n = 600001
+    ln = np.full(n, 3, np.int64)
+    if kind.startswith("long"):
+        ln[{"long_first": 0, "long_mid": n // 2, "long_last": n - 1}[kind]] = 97
+    elif kind == "runs":
+        ln[(np.arange(n) // 1000) % 16 == 0] = 48
+    else:
+        ln[:] = 5
+        ln[-200:] = 0
+    return ln
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("kind", ["long_first", "long_mid", "long_last", "runs", "empty_end"])
+def test_row_patterns_of_uneven_rows(m, ctx, oracle, kind, dtype):
+    """Block plans of matrices with few row patterns and uneven rows, where a
+    block's LDS is sized for the fullest block of the matrix: the CPU row
+    loop's bits under the plan made at upload and under row patterns where
+    they are taken."""
+    say("uneven rows", kind, dtype.__name__)
+    ln = _uneven(kind)
+    rows = ln.size
+    rp = np.zeros(rows + 1, np.int32)
+    np.cumsum(ln, out=rp[1:])
+    ci = (np.repeat(np.arange(rows) - rp[:-1], ln) + np.arange(rp[-1])).astype(np.int32)
+    val = np.random.default_rng(8).uniform(-1, 1, ci.size).astype(dtype)
+    cols = rows + 100
+    x = oracle.random_vector(cols, -1.0, 1.0, 40, dtype=dtype)
+    ref = oracle.spmv(rp, ci, val, x)
+    A = m.CRS(ctx, rows, cols, rp, ci, val)
+    X, Y = m.Vector(ctx, x, dtype=dtype), m.Vector(ctx, n=rows, dtype=dtype)
+    m.matvec(A, X, Y)
+    assert bits_equal(Y.download(), ref)
+    if kind == "runs":  # most of the LDS would be empty
+        with pytest.raises(m.MgxError):
+            A.set_plan(row_walk=4)
+    else:
+        A.set_plan(row_walk=4)
+    Y.fill(3.0)
+    m.matvec(A, X, Y)
+    assert bits_equal(Y.download(), ref)
+    for o in (A, X, Y):
         o.free()
 
 
