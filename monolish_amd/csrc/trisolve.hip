@@ -744,6 +744,22 @@ void build_tri_plan(const std::vector<int32_t> &ptr, const std::vector<int32_t> 
   };
   const int nthr = n < 65536 ? 1 : 4;
   std::vector<Part> part(nthr);
+  // the rows of a level, in a wave, run in any order: those of one batch's
+  // width first, longer ones by their length, so that a batch is not cut at
+  // every change between them (2000-row M-matrix, half of its rows longer
+  // than 14 entries: 0.89 -> 0.29 ms an iteration of SOR-PCG)
+  auto sort_levels = [&](int64_t k0, int64_t k1) {
+    for (int64_t k = k0; k < k1;) {
+      int64_t e = k;
+      bool lng = false;
+      for (; e < k1 && lev[order[e]] == lev[order[k]]; e++) lng = lng || cnt[order[e]] > D;
+      if (lng)
+        std::stable_sort(order.begin() + k, order.begin() + e, [&](int32_t x, int32_t y) {
+          return std::max(cnt[x], D) < std::max(cnt[y], D);
+        });
+      k = e;
+    }
+  };
   auto work = [&](int64_t v0, int64_t v1, Part &out) {
     std::vector<int4> &hdr = out.hdr;
     std::vector<uint16_t> &slot = out.slot;
@@ -763,6 +779,7 @@ void build_tri_plan(const std::vector<int32_t> &ptr, const std::vector<int32_t> 
       wv[2] = std::min<int64_t>(v * srows, n);
       wv[3] = (int64_t)ext.size();
       const int64_t k1 = std::min<int64_t>(wv[2] + srows, n);
+      sort_levels(wv[2], k1);
       const int64_t base = v / kChWaves * P.crows;  // the chunk's first sweep position
       const uint32_t ring0 = (uint32_t)P.crows + (uint32_t)(v % kChWaves) * kRing;
       int64_t ntaken = 0;

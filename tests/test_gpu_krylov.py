@@ -827,7 +827,7 @@ def _banded(n, band, per_row, seed):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("name", ["grid5", "grid7", "grid7_wide", "banded", "dense_rows",
-                                  "scattered", "scattered_wide"])
+                                  "scattered_small", "scattered", "scattered_wide"])
 def test_sweeps_across_chunks_bit_exact(m, ctx, oracle, name, dtype):
     """Triangular sweeps over several chunks of rows, at each width of the
     batches (2, 4, 8 and 14 entries a row, rows of many more), with long and
@@ -839,6 +839,7 @@ def test_sweeps_across_chunks_bit_exact(m, ctx, oracle, name, dtype):
                    "grid7_wide": lambda: m.stencil3d(70, 61, 63, 7, 0.1),
                    "banded": lambda: _banded(20011, 3000, 7, 1),
                    "dense_rows": lambda: _banded(9001, 8700, 40, 2),
+                   "scattered_small": lambda: m.mmatrix(2000),
                    "scattered": lambda: m.mmatrix(20000),
                    "scattered_wide": lambda: m.mmatrix(140001)}[name]()
     val = val.astype(dtype)
