@@ -56,16 +56,35 @@ constexpr int kRing = 1024;      // values of earlier chunks that a wave keeps
 // ms; 3D 27-point 96^3 (1328) 2.06 / 1.87 / 1.68 ms, 128^3 (2356) 2.86 /
 // 2.58 / 2.36 ms, 7-point 100^3 (3356) 0.95 / 0.82 / 0.77 ms.
 constexpr int kWaveRows = 2048, kWaveRowsWide = 256, kWideLevel = 1000;
-// Scattered matrices: a chunk of 8192 rows reads more than kScattered
-// distinct values of earlier chunks per row and wave (grids: up to 1.3).  The
-// dependency-driven form takes them when their levels can fill the chip (at
-// least kFlowMinRows rows, kFlowMinWidth a level): 300000-row random
-// M-matrix, 5085 rows a level, 0.65 ms an iteration against 1.77 ms in
-// chunks.  Smaller ones run in chunks of kWaveRowsScattered rows a wave:
-// 20000 rows, 0.69 ms.
-constexpr double kScattered = 3.0;
+// Matrices whose rows read scattered rows gain less from chunks, or lose: the
+// chain then crosses a chunk at almost every level, and a batch is cut short
+// by the values of earlier chunks that it takes.  model_share runs the
+// schedule of kModelRows rows from the middle, with what a batch, a level and
+// a value's way measured, and sets it against kFlowLevelUs for each level of
+// those rows, what one costs in the dependency-driven form: grids come to
+// 0.09-0.2 of it, rows that read random rows of a band to 0.33-1.1, of the
+// whole matrix to 1.4 and more.  From kScattered on a wave gets few rows, from
+// kFlowBetter on the dependency-driven form runs where there are kFlowRows
+// rows, kFlowMinWidth a level on average, and kFlowMinLevels levels (with
+// fewer the entries take longer than the chain).  Per SOR-PCG iteration, FP64,
+// in us, with 2048 / 256 / 64 rows a wave / dependency-driven:
+//   band of 1000, 300000 rows (74 a level), share 0.33-0.43
+//                                            11403 / 12522 / 24084 / 26392
+//   band of 3000, 20000 rows (290), 0.75         567 / 516 / 500 / 565
+//   band of 5000, 50000 rows (485), 1.0         1146 / 884 / 884 / 789
+//   band of 5000, 200000 rows (350), 0.6-0.8   5464 / 4558 / 7150 / 4386
+//   M-matrix, 20000 rows (400), 1.4             1371 / 700 / 560 / 559
+//   M-matrix, 130000 rows (2321), 1.7          2987 / 1007 / 1254 / 696
+//   M-matrix of 60 entries a row, 20000 rows (136), 3.9
+//                                              4706 / 2651 / 1799 / 2078
+//   5-point 700^2, rows permuted (13 levels), 1.0   501 / 352 / 482 / 426
 constexpr int kWaveRowsScattered = 64;
-constexpr int64_t kFlowMinRows = 1 << 17, kFlowMinWidth = 256;
+constexpr int64_t kModelRows = 4096, kFlowRows = 32768, kFlowMinWidth = 256;
+constexpr int kFlowMinLevels = 32;
+constexpr double kScattered = 0.42, kFlowBetter = 0.6, kFlowLevelUs = 3.6;
+// a batch, a level (and each of its entries' width), a value from an earlier
+// chunk and from another wave of the chunk, in us
+constexpr double kBatchUs = 0.73, kLevelUs = 0.11, kEntryUs = 0.023, kFarUs = 2.8, kNearUs = 0.09;
 constexpr uint64_t kSpinTicks = 200000000;  // 2 s of the 100 MHz clock without progress
 
 // batch header: x, y = lanes whose row starts a level, z = rows | values of
@@ -378,7 +397,7 @@ __global__ __launch_bounds__(64 * kChWaves) void k_tri_chunk(const TriArgs<T> a)
 }
 
 // The dependency-driven form, for matrices whose rows read scattered rows
-// all over the matrix (kScattered): hardly any dependency stays inside a
+// (kFlowBetter): hardly any dependency stays inside a
 // chunk there, and what bounds the sweep is the number of values fetched.
 // Persistent waves take 64 consecutive level-order positions at a time from
 // a ticket counter and each lane computes its row as soon as the rows it
@@ -452,7 +471,7 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
             a[u] = dcoef[e];
           }
 #pragma unroll
-          // plain loads: out held kEmpty when this kernel started (k_flow_init,
+          // plain loads: out held kEmpty when this kernel started (k_tri_init,
           // an earlier kernel of the stream) and changes once, to the final
           // value, so a cached copy is either that value or a stale kEmpty,
           // which the device-coherent poll below resolves
@@ -614,6 +633,68 @@ void push_values(std::vector<int4> &hdr, std::vector<int32_t> &ext,
 
 bool dep_of(int filter, int64_t i, int32_t c) { return filter == 2 ? c > i : c < i; }
 
+// the time of the sweep over positions [p0, p0 + pn) in chunks of kChWaves
+// waves of srows rows (p0 a multiple of them), as a share of what the
+// dependency-driven form takes for the levels of these rows.  for_reads(p, f)
+// calls f with each position that position p reads (values from before p0
+// are there); lev and cnt by position
+template <class Lev, class Cnt, class Reads>
+double model_share(int64_t n, int64_t p0, int64_t pn, int64_t srows, int D, int maxnew, Lev lev,
+                   Cnt cnt, Reads for_reads) {
+  std::vector<int32_t> depth(pn, 0), stamp(n, -1);
+  int32_t levels = 1;
+  for (int64_t p = p0; p < p0 + pn; p++) {
+    int32_t d = 0;
+    for_reads(p, [&](int64_t q) { if (q >= p0) d = std::max(d, depth[q - p0] + 1); });
+    depth[p - p0] = d;
+    levels = std::max(levels, d + 1);
+  }
+  std::vector<double> done(pn, 0.0);
+  std::vector<int64_t> ord;
+  double end = 0;
+  int32_t v = 0;
+  for (int64_t a = p0; a < p0 + pn; a += srows, v++) {
+    const int64_t b = std::min(a + srows, p0 + pn), base = a - v % kChWaves * srows;
+    ord.resize(b - a);
+    for (int64_t p = a; p < b; p++) ord[p - a] = p;
+    std::stable_sort(ord.begin(), ord.end(), [&](int64_t x, int64_t y) {
+      return std::make_pair(lev(x), std::max(cnt(x), D)) < std::make_pair(lev(y), std::max(cnt(y), D));
+    });
+    double now = 0;
+    for (size_t k = 0; k < ord.size();) {
+      const bool lng = cnt(ord[k]) > D;
+      size_t e = k;
+      int fresh = 0, longest = 0;
+      while (e < ord.size() && e - k < 64) {
+        const int64_t p = ord[e];
+        if ((cnt(p) > D) != lng || (lng && lev(p) != lev(ord[k]))) break;
+        int news = 0;
+        for_reads(p, [&](int64_t q) { news += q < base && stamp[q] != v; });
+        if (e > k && fresh + news > maxnew) break;
+        for_reads(p, [&](int64_t q) { if (q < base) stamp[q] = v; });
+        fresh += news;
+        longest = std::max(longest, cnt(p));
+        e++;
+      }
+      const int parts = std::max(1, (longest + D - 1) / D);
+      now += kBatchUs * parts;
+      while (k < e) {
+        const int32_t l = lev(ord[k]);
+        const size_t k0 = k;
+        double in = 0;
+        for (; k < e && lev(ord[k]) == l; k++)
+          for_reads(ord[k], [&](int64_t q) {
+            if (q >= p0 && q < a) in = std::max(in, done[q - p0] + (q < base ? kFarUs : kNearUs));
+          });
+        now = std::max(now, in) + (kLevelUs + kEntryUs * D) * parts;
+        for (size_t u = k0; u < k; u++) done[ord[u] - p0] = now;
+      }
+    }
+    end = std::max(end, now);
+  }
+  return end / (kFlowLevelUs * levels);
+}
+
 }  // namespace
 
 void build_tri_plan(const std::vector<int32_t> &ptr, const std::vector<int32_t> &col,
@@ -657,28 +738,37 @@ void build_tri_plan(const std::vector<int32_t> &ptr, const std::vector<int32_t> 
   P.n = n;
   P.rev = filter == 2;
   auto at = [&](int64_t i) { return P.rev ? n - 1 - i : i; };  // sweep position of row i
-  // scattered? (distinct values of earlier chunks in a sample of waves)
-  bool scattered = false;
+  // entries per row and batch: the smallest width that takes 98 % of the rows
+  // in one batch (2, 3 and 13 entries on 5-, 7- and 27-point grids)
   {
-    const int64_t span = (int64_t)kChWaves * kWaveRows, nw = n / kWaveRows;
-    const int64_t step = std::max<int64_t>(1, nw / 32);
-    std::vector<int64_t> seen(nw > kChWaves ? n : 0, -1);
-    int64_t nrows = 0, far = 0;
-    for (int64_t v = kChWaves; v < nw; v += step) {
-      const int64_t base = v * kWaveRows / span * span;
-      for (int64_t p = v * kWaveRows; p < (v + 1) * kWaveRows; p++)
-        for_deps(at(p), [&](int32_t j) {
-          if (at(col[j]) < base && seen[col[j]] != v) seen[col[j]] = v, far++;
-        });
-      nrows += kWaveRows;
-    }
-    scattered = (double)far > kScattered * (double)nrows;
+    const int widths[4] = {2, 4, 8, 14};
+    int64_t over[4] = {0, 0, 0, 0};
+    for (int64_t i = 0; i < n; i++)
+      for (int q = 0; q < 4; q++) over[q] += cnt[i] > widths[q];
+    int q = 0;
+    while (q < 3 && over[q] * 50 > n) q++;
+    P.width = widths[q];
+  }
+  const int D = P.width;
+  const WidthSizes wd = D == 2   ? width_sizes<2>()
+                        : D == 4 ? width_sizes<4>()
+                        : D == 8 ? width_sizes<8>()
+                                 : width_sizes<14>();
+  const int maxnew = 64 * wd.far;
+  double share = 0;  // (more than a chunk's rows, or nothing is handed over)
+  if (n > kChWaves * kWaveRows) {
+    const int64_t pn = std::min(n, kModelRows), span = kChWaves * kWaveRowsWide;
+    share = model_share(
+        n, (n - pn) / 2 / span * span, pn, kWaveRowsWide, D, maxnew,
+        [&](int64_t p) { return lev[at(p)]; }, [&](int64_t p) { return cnt[at(p)]; },
+        [&](int64_t p, auto &&f) { for_deps(at(p), [&](int32_t j) { f(at(col[j])); }); });
   }
   P.d_ticket = (uint32_t *)dev_alloc(256);  // [0] ticket, [1] stall flag, [2] batches done
   MGX_HIP(hipMemset(P.d_ticket, 0, 256));
   L.d_rows = upload(rows);
   L.d_ptr = upload(L.ptr);
-  P.flow = scattered && n >= kFlowMinRows && n >= kFlowMinWidth * (int64_t)nlev;
+  P.flow = n >= kFlowRows && share >= kFlowBetter && nlev >= kFlowMinLevels &&
+           n >= kFlowMinWidth * (int64_t)nlev;
   if (P.flow) {
     int64_t nd = 0;
     for (int64_t i = 0; i < n; i++) nd += cnt[i];
@@ -704,9 +794,9 @@ void build_tri_plan(const std::vector<int32_t> &ptr, const std::vector<int32_t> 
   }
   // rows of each wave in level order
   const int64_t per = (n + kChWaves - 1) / kChWaves;
-  const int64_t cap = scattered                             ? kWaveRowsScattered
-                      : n >= kWideLevel * (int64_t)nlev ? kWaveRowsWide
-                                                            : kWaveRows;
+  const int64_t cap = share >= 1 && n < kFlowRows ? kWaveRowsScattered
+                      : share >= kScattered || n >= kWideLevel * (int64_t)nlev ? kWaveRowsWide
+                                                                             : kWaveRows;
   const int64_t srows = std::min<int64_t>(cap, std::max<int64_t>(64, (per + 63) / 64 * 64));
   P.crows = (int32_t)(kChWaves * srows);
   P.nchunk = (int32_t)((n + P.crows - 1) / P.crows);
@@ -717,24 +807,7 @@ void build_tri_plan(const std::vector<int32_t> &ptr, const std::vector<int32_t> 
     for (int64_t v = 0; v < nwave; v++) next[v] = (int32_t)std::min<int64_t>(v * srows, n);
     for (int64_t k = 0; k < n; k++) order[next[at(rows[k]) / srows]++] = rows[k];
   }
-  // entries per row and batch: the smallest width that takes 98 % of the rows
-  // in one batch (2, 3 and 13 entries on 5-, 7- and 27-point grids)
-  {
-    const int widths[4] = {2, 4, 8, 14};
-    int64_t over[4] = {0, 0, 0, 0};
-    for (int64_t i = 0; i < n; i++)
-      for (int q = 0; q < 4; q++) over[q] += cnt[i] > widths[q];
-    int q = 0;
-    while (q < 3 && over[q] * 50 > n) q++;
-    P.width = widths[q];
-  }
   const uint16_t zero = (uint16_t)slot_zero((uint32_t)P.crows);
-  const int D = P.width;
-  const WidthSizes wd = D == 2   ? width_sizes<2>()
-                        : D == 4 ? width_sizes<4>()
-                        : D == 8 ? width_sizes<8>()
-                                 : width_sizes<14>();
-  const int maxnew = 64 * wd.far;
   std::vector<int64_t> wave((nwave + 1) * 4);
   // the waves' batches, by a few threads, each for a run of waves
   struct Part {

@@ -827,7 +827,7 @@ def _banded(n, band, per_row, seed):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("name", ["grid5", "grid7", "grid7_wide", "banded", "dense_rows",
-                                  "scattered_small", "scattered", "scattered_wide"])
+                                  "scattered_small", "scattered", "scattered_wide", "wide_band"])
 def test_sweeps_across_chunks_bit_exact(m, ctx, oracle, name, dtype):
     """Triangular sweeps over several chunks of rows, at each width of the
     batches (2, 4, 8 and 14 entries a row, rows of many more), with long and
@@ -841,7 +841,8 @@ def test_sweeps_across_chunks_bit_exact(m, ctx, oracle, name, dtype):
                    "dense_rows": lambda: _banded(9001, 8700, 40, 2),
                    "scattered_small": lambda: m.mmatrix(2000),
                    "scattered": lambda: m.mmatrix(20000),
-                   "scattered_wide": lambda: m.mmatrix(140001)}[name]()
+                   "scattered_wide": lambda: m.mmatrix(140001),
+                   "wide_band": lambda: _banded(40001, 6000, 4, 3)}[name]()
     val = val.astype(dtype)
     n = len(rp) - 1
     b = oracle.random_vector(n, -1.0, 1.0, 91, dtype=dtype)
