@@ -61,7 +61,7 @@ __device__ __forceinline__ void tile_spmv(const SysDesc<T> &d, int64_t tile,
     if (d0 < 0) {
       const int32_t e0 = d.rp[ra], e1 = d.rp[ra + 1];
       T s = 0;
-      for (int32_t e = e0 + t; e < e1; e += kBlock) {
+      for (uint32_t e = e0 + t; e < (uint32_t)e1; e += kBlock) {
         T pr = d.val[e] * gv(d.ci[e]);
         s = s + pr;
       }
@@ -1267,7 +1267,7 @@ __global__ __launch_bounds__(kBlock) void k_setup_diag(const SysDesc<T> *sys,
     best[t] = -1;
     __syncthreads();
     const int32_t e0 = srp[0], e1 = srp[nr];
-    for (int32_t j = e0 + t; j < e1; j += kBlock) {
+    for (uint32_t j = e0 + t; j < (uint32_t)e1; j += kBlock) {
       int lo = 0, hi = nr - 1;
       while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;

@@ -356,12 +356,14 @@ __device__ __forceinline__ void stream_products(const T *__restrict__ val,
   typedef T VT __attribute__((ext_vector_type(W)));
   typedef int32_t VI __attribute__((ext_vector_type(W)));
   const int32_t ea = e0 & ~(W - 1);
+  // unsigned, here and in the other loops over entries: positions past the
+  // last one may be 2^31 or more
   VT v[U];
   VI c[U];
 #pragma unroll
   for (int k = 0; k < U; k++) {
-    const int32_t base = ea + ((int32_t)threadIdx.x + k * kBlock) * W;
-    if (base < e1) {
+    const uint32_t base = ea + (threadIdx.x + k * kBlock) * W;
+    if (base < (uint32_t)e1) {
       v[k] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(val + base));
       c[k] = __builtin_nontemporal_load(reinterpret_cast<const VI *>(ci + base));
     }
@@ -369,17 +371,18 @@ __device__ __forceinline__ void stream_products(const T *__restrict__ val,
   T xv[U][W];
 #pragma unroll
   for (int k = 0; k < U; k++) {
-    const int32_t base = ea + ((int32_t)threadIdx.x + k * kBlock) * W;
+    const uint32_t base = ea + (threadIdx.x + k * kBlock) * W;
 #pragma unroll
     for (int j = 0; j < W; j++)
-      if (base + j >= e0 && base + j < e1) xv[k][j] = gv(c[k][j]);
+      if (base + j >= (uint32_t)e0 && base + j < (uint32_t)e1) xv[k][j] = gv(c[k][j]);
   }
 #pragma unroll
   for (int k = 0; k < U; k++) {
-    const int32_t base = ea + ((int32_t)threadIdx.x + k * kBlock) * W;
+    const uint32_t base = ea + (threadIdx.x + k * kBlock) * W;
 #pragma unroll
     for (int j = 0; j < W; j++)
-      if (base + j >= e0 && base + j < e1) prod[base + j - e0] = (T)v[k][j] * xv[k][j];
+      if (base + j >= (uint32_t)e0 && base + j < (uint32_t)e1)
+        prod[base + j - e0] = (T)v[k][j] * xv[k][j];
   }
 }
 

@@ -49,7 +49,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(
   const int32_t e0 = d0.y, e1 = d1.y;
   if (d0.x < 0) {
     T s = 0;
-    for (int32_t e = e0 + (int32_t)threadIdx.x; e < e1; e += kBlock) {
+    for (uint32_t e = e0 + threadIdx.x; e < (uint32_t)e1; e += kBlock) {
       T p = val[e] * x[ci[e]];
       s = s + p;
     }
@@ -98,16 +98,16 @@ __global__ __launch_bounds__(kBlock) void k_spmv(
       VI c[G];
 #pragma unroll
       for (int k = 0; k < G; k++) {
-        const int32_t base = ea + ((int32_t)threadIdx.x + (k0 + k) * kBlock) * W;
-        if (k0 + k < U && base < e1) {
+        const uint32_t base = ea + (threadIdx.x + (k0 + k) * kBlock) * W;
+        if (k0 + k < U && base < (uint32_t)e1) {
           v[k] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(val + base));
           c[k] = __builtin_nontemporal_load(reinterpret_cast<const VI *>(ci + base));
         }
       }
 #pragma unroll
       for (int k = 0; k < G; k++) {
-        const int32_t base = ea + ((int32_t)threadIdx.x + (k0 + k) * kBlock) * W;
-        if (k0 + k < U && base < e1) {
+        const uint32_t base = ea + (threadIdx.x + (k0 + k) * kBlock) * W;
+        if (k0 + k < U && base < (uint32_t)e1) {
           *reinterpret_cast<VT *>(sv + (base - ea)) = v[k];
           *reinterpret_cast<VI *>(sc + (base - ea)) = c[k];
         }
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_longrows(
   const int32_t r0 = rows[blockIdx.x];
   const int32_t e0 = rp[r0], e1 = rp[r0 + 1];
   T s = 0;
-  for (int32_t e = e0 + (int32_t)threadIdx.x; e < e1; e += kBlock) {
+  for (uint32_t e = e0 + threadIdx.x; e < (uint32_t)e1; e += kBlock) {
     T p = val[e] * x[ci[e]];
     s = s + p;
   }
@@ -640,7 +640,7 @@ __global__ __launch_bounds__(kBlock) void k_diag(int64_t n, const int32_t *__res
   best[t] = -1;
   __syncthreads();
   const int32_t e0 = srp[0], e1 = srp[nr];
-  for (int32_t j = e0 + t; j < e1; j += kBlock) {
+  for (uint32_t j = e0 + t; j < (uint32_t)e1; j += kBlock) {
     // largest local row lr with srp[lr] <= j
     int lo = 0, hi = nr - 1;
     while (lo < hi) {

@@ -795,7 +795,7 @@ def test_entry_positions_next_to_2_31(m, ctx):
     X, Y = m.Vector(ctx, x, dtype=np.float32), m.Vector(ctx, n=rows, dtype=np.float32)
     c = np.concatenate([[0], np.cumsum(x.astype(np.int64))])
     ref = (c[L:L + rows] - c[:rows]).astype(np.float32)
-    for plan in (None,):
+    for plan in (None, dict(row_walk=0), dict(row_walk=1, nnz_per_block=4096)):
         if plan:
             A.set_plan(**plan)
         Y.fill(-1.0)
