@@ -727,6 +727,35 @@ def test_row_patterns_of_uneven_rows(m, ctx, oracle, kind, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_row_patterns_with_nan_and_inf(m, ctx, oracle, dtype):
+    """NaN and infinities in x and in the values under row patterns: they
+    reach the rows that hold them and no other (no lane adds what lies beside
+    its row)."""
+    say("patterns with nan and inf", dtype.__name__)
+    rng = np.random.default_rng(3)
+    rows = 150001
+    rp, ci, cols = pattern_rows(rng, rows, 7, (12, 11, 13, 10), 40)
+    val = rng.uniform(-1, 1, rp[-1]).astype(dtype)
+    val[rng.integers(rp[-1], size=300)] = np.inf
+    val[rng.integers(rp[-1], size=300)] = np.nan
+    x = oracle.random_vector(cols, -1.0, 1.0, 40, dtype=dtype)
+    x[rng.integers(cols, size=300)] = -np.inf
+    x[rng.integers(cols, size=300)] = np.nan
+    ref = oracle.spmv(rp, ci, val, x)
+    bad = np.isnan(ref)
+    assert 1000 < bad.sum() < rows // 2 and np.isinf(ref).any()
+    A = m.CRS(ctx, rows, cols, rp, ci, val)
+    X, Y = m.Vector(ctx, x, dtype=dtype), m.Vector(ctx, n=rows, dtype=dtype)
+    for walk in (4, 2):
+        A.set_plan(row_walk=walk)
+        m.matvec(A, X, Y)
+        y = Y.download()
+        assert np.array_equal(np.isnan(y), bad) and bits_equal(y[~bad], ref[~bad]), walk
+    for o in (A, X, Y):
+        o.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_block_plans_of_a_matrix_with_row_patterns(m, oracle, dtype):
     """Block plans that the program chooses, on a matrix that starts with row
     patterns: the products-staged kernel in blocks of any size, the pattern

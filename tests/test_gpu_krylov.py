@@ -216,10 +216,12 @@ def test_cg_persistent_kernel(m, ctx, oracle, blocks):
     """The fused CG of one small system in one cooperative launch (blocks=1:
     a grid of one block per 128-row quarter; 7, 64: capped grids, blocks own
     several quarters; 0: one launch per stage) is bit-identical to the
-    oracle, including the maxiter and NaN exits."""
+    oracle, including the maxiter and NaN exits.  Rows of 27 entries: none of
+    these solves is resident (one would raise here)."""
     say("cg persistent", blocks)
-    rp, ci, val = _poisson(oracle, 60)  # n = 3600: 8 tiles, 32 quarters
+    rp, ci, val = m.stencil3d(15, 16, 15, 27, 1e-2)  # n = 3600: 8 tiles, 29 quarters
     n = len(rp) - 1
+    resident_hook(m, ctx, 0)
     b = oracle.random_vector(n, -1.0, 1.0, 1001)
     tol = 1e-10 * float(oracle.nrm2(b))
     m.set_persistent(ctx, blocks != 0, max_blocks=blocks)
@@ -238,6 +240,7 @@ def test_cg_persistent_kernel(m, ctx, oracle, blocks):
         assert res.status == m.SOLVER_RESIDUAL_NAN and res.final_iter == 1
     finally:
         m.set_persistent(ctx, False)
+        resident_hook(m, ctx)
 
 
 def _ring(n, reach, seed):
@@ -865,6 +868,46 @@ def test_sweeps_across_chunks_bit_exact(m, ctx, oracle, name, dtype):
     assert res.status == ref[0] and res.final_iter == ref[2]
     assert bits_equal(x, ref[1])
     assert bits_equal(res.rhistory, ref[4])
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("name", ["grid5", "grid7", "grid27", "scattered", "flow", "arrow"])
+def test_sweeps_with_nan_and_inf(m, ctx, oracle, name, dtype):
+    """NaN and infinities in the right-hand side of a sweep: the rows that they
+    reach look again at every value they read (a missing one is a NaN too),
+    and none waits for one that is there.  The oracle's values, its infinities
+    and NaNs in the same rows, in chunks at each width and in the
+    dependency-driven form; two systems in one matrix, one of them clean."""
+    import scipy.sparse as sp
+    one = {"grid5": lambda: m.laplacian2d(193, 101),
+           "grid7": lambda: m.stencil3d(33, 35, 37, 7, 0.1),
+           "grid27": lambda: m.stencil3d(25, 23, 27, 27, 0.1),
+           "scattered": lambda: m.mmatrix(6000),
+           "flow": lambda: m.mmatrix(20001),
+           "arrow": lambda: _arrow(9001)}[name]()
+    half = len(one[0]) - 1
+    M = sp.csr_matrix((one[2], one[1], one[0]), shape=(half, half))
+    M = sp.csr_matrix(sp.block_diag((M, M)))
+    M.sort_indices()
+    rp, ci = M.indptr.astype(np.int32), M.indices.astype(np.int32)
+    val = M.data.astype(dtype)
+    n = len(rp) - 1
+    say("nan sweeps", name, dtype.__name__, n)
+    A, X = m.CRS(ctx, n, n, rp, ci, val), m.Vector(ctx, n=n, dtype=dtype)
+    for at, what in ((half // 3, np.nan), (n - 2, np.nan), (half + 1, np.inf), (0, -np.inf)):
+        b = oracle.random_vector(n, -1.0, 1.0, 91, dtype=dtype)
+        b[at] = what
+        rc, ref = oracle.ilu_precond(rp, ci, val, 5, b)
+        assert rc == 0
+        B = m.Vector(ctx, b, dtype=dtype)
+        assert m.ilu_solve(A, X, B).status == 0
+        x = X.download()
+        assert np.array_equal(np.isnan(x), np.isnan(ref)), (at, what)
+        ok = ~np.isnan(ref)
+        assert ok.sum() >= half and bits_equal(x[ok], ref[ok]), (at, what)
+        B.free()
+    for v in (A, X):
+        v.free()
 
 
 def _wide_then_chain(n_free, n_chain):
