@@ -782,11 +782,12 @@ void spmv_plan_build_with(Csr *A, const int32_t *rp, int rows_req, int nnz_req, 
   const int64_t nb = (int64_t)blk.size();
   blk.push_back(make_int2((int32_t)rows, rp[rows]));
   A->plan.rows32 = 0;
-  for (int64_t i = 0; i < rows; i++) {
-    const int32_t len = rp[i + 1] - rp[i];
-    A->plan.rows32 += len > 0 && len % 32 == 0;
-  }
-  for (int k = 0; k < 2; k++) {
+  if (A->d_pat && mx / 32 * 32 >= std::max(mn, 32))  // (no other row can count)
+    for (int64_t i = 0; i < rows; i++) {
+      const int32_t len = rp[i + 1] - rp[i];
+      A->plan.rows32 += len > 0 && len % 32 == 0;
+    }
+  for (int k = 0; k < 2 && A->d_pat; k++) {
     const int64_t step = k ? kBlock : kBlock / 2;
     int32_t most = 0;
     for (int64_t i = 0; i < rows; i += step)
