@@ -172,9 +172,9 @@ struct SpmvPlan {
   int32_t walk = 0;      // stream blocks: 0 product-staged, 1 row walk
   double mean_row = 0;
   // most entries of 128 and of 256 rows from a multiple of 128 / 256 on, and
-  // rows of 32, 64, ... entries (row patterns)
+  // rows of 32, 48, 64, ... entries (row patterns)
   int32_t block_ent[2] = {0, 0};
-  int64_t rows32 = 0;
+  int64_t rows_bank = 0;
   int32_t rowpat = 0;    // block plan of a matrix with row patterns: values
                          // staged, columns from the patterns (walk unused)
   double tuned_us = 0;   // SpMV time measured by the autotuner (0: not tuned)

@@ -718,17 +718,21 @@ static size_t rowpat_bytes(const Csr *A, int rows, size_t es) {
 // rows of a k_spmv_pat block: kBlock, or half of that where it would take more
 // than 32 KB of LDS and leave a compute unit few wavefronts (27-point 128^3
 // FP64, 59 KB: 118 us with 256 rows, 112 with 128; 16 entries a row, 33 KB:
-// 31.5 / 30.2; 27-point FP32, 31 KB: 52 / 58); 0: not even that fits, or most
-// rows start in the same bank (rows of 32 entries, FP64: products staged 94.7,
-// this 100.3), or rows of uneven length leave most of that LDS empty: where
-// LDS limits the blocks of a compute unit, they have to keep 32 KB of values
-// in flight (runs of 1000 rows of 48 entries among rows of 3, 18 KB: products
-// staged 16.2, this 28.2 us in FP64, 13.9 / 15.3 in FP32)
+// 31.5 / 30.2; 27-point FP32, 31 KB: 52 / 58); 0 (products staged instead):
+// - a compute unit would not hold four of the smaller blocks, 40 KB each (16 M
+//   entries, FP64, products staged / this, in us: rows of 34 entries, 40 KB,
+//   39.0 / 36.3; of 40, 46 KB, 40.5 / 41.7; of 47, 57 KB, 39.8 / 47.8);
+// - most rows start in few banks (rows of 32 entries, FP64, 94.7 / 100.3; of
+//   48, 46.7 / 53.1, FP32 27.3 / 31.1);
+// - rows of uneven length leave most of that LDS empty: where LDS limits the
+//   blocks of a compute unit, they have to keep 32 KB of values in flight
+//   (runs of 1000 rows of 48 entries among rows of 3, 18 KB: 16.2 / 28.2 in
+//   FP64, 13.9 / 15.3 in FP32)
 static int rowpat_rows(const Csr *A, size_t es) {
-  if (2 * A->plan.rows32 > A->rows) return 0;
+  if (2 * A->plan.rows_bank > A->rows) return 0;
   for (int rb : {kBlock, kBlock / 2}) {
     const size_t lds = rowpat_bytes(A, rb, es), fit = ((size_t)160 << 10) / lds;
-    if (lds > (rb == kBlock ? 32768u : 65536u)) continue;
+    if (lds > (rb == kBlock ? 32768u : 40960u)) continue;
     if (fit * rb >= 2048 || (double)(fit * rb * es) * A->plan.mean_row >= 32768) return rb;
   }
   return 0;
@@ -781,11 +785,11 @@ void spmv_plan_build_with(Csr *A, const int32_t *rp, int rows_req, int nnz_req, 
   }
   const int64_t nb = (int64_t)blk.size();
   blk.push_back(make_int2((int32_t)rows, rp[rows]));
-  A->plan.rows32 = 0;
-  if (A->d_pat && mx / 32 * 32 >= std::max(mn, 32))  // (no other row can count)
+  A->plan.rows_bank = 0;
+  if (A->d_pat && mx / 16 * 16 >= std::max(mn, 32))  // (no other row can count)
     for (int64_t i = 0; i < rows; i++) {
       const int32_t len = rp[i + 1] - rp[i];
-      A->plan.rows32 += len > 0 && len % 32 == 0;
+      A->plan.rows_bank += len >= 32 && len % 16 == 0;
     }
   for (int k = 0; k < 2 && A->d_pat; k++) {
     const int64_t step = k ? kBlock : kBlock / 2;

@@ -634,9 +634,9 @@ def pattern_rows(rng, rows, npat, lens, span):
     (70001, 61, (64, 63, 61), 90),   # and 61 do not fit it
     (100001, 2, (16, 16), 40),       # FP64: 32 KB of LDS are not enough for 256 rows
     (100127, 2, (15, 14), 40),       # and are for these
-    (100129, 3, (63, 62, 61), 90),   # FP64: 128 rows take just under 64 KB
-    (100130, 3, (65, 64, 63), 90),   # and just over
-    (60001, 4, (32, 31, 30), 90),    # rows 32 apart in LDS: columns from memory
+    (100129, 3, (39, 38, 37), 90),   # FP64: 128 rows take just under 40 KB
+    (100130, 3, (41, 40, 39), 90),   # and just over
+    (60001, 4, (48, 48, 30), 90),    # most rows 48 apart in LDS: columns from memory
 ])
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_sliced_row_patterns(m, ctx, oracle, dtype, rows, npat, lens, span):
