@@ -697,8 +697,23 @@ double model_share(int64_t n, int64_t p0, int64_t pn, int64_t srows, int D, int 
 
 }  // namespace
 
+static void plan_free(TriPlan &P) {
+  levels_free(P.lev);
+  dev_free(P.d_hdr);
+  dev_free(P.d_rec);
+  dev_free(P.d_dcol);
+  dev_free(P.d_slot);
+  dev_free(P.d_dent);
+  dev_free(P.d_ext);
+  dev_free(P.d_row);
+  dev_free(P.d_wave);
+  dev_free(P.d_ticket);
+  P = TriPlan();
+}
+
 void build_tri_plan(const std::vector<int32_t> &ptr, const std::vector<int32_t> &col,
                     const std::vector<int32_t> *ent, int64_t n, int filter, TriPlan &P) {
+  plan_free(P);  // (what a build that ran out of memory left)
   // dependency entries of each row, in the row's order (filter 1 stops at
   // the first entry that is not left of the diagonal)
   std::vector<int32_t> cnt(n, 0), lev(n, 0);
@@ -1073,19 +1088,7 @@ void levels_free(SorLevels &L) {
 }
 
 void tri_free(Csr *A) {
-  for (TriPlan &P : A->tri) {
-    levels_free(P.lev);
-    dev_free(P.d_hdr);
-    dev_free(P.d_rec);
-    dev_free(P.d_dcol);
-    dev_free(P.d_slot);
-    dev_free(P.d_dent);
-    dev_free(P.d_ext);
-    dev_free(P.d_row);
-    dev_free(P.d_wave);
-    dev_free(P.d_ticket);
-    P = TriPlan();
-  }
+  for (TriPlan &P : A->tri) plan_free(P);
 }
 
 }  // namespace mgx
