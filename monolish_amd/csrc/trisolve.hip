@@ -397,22 +397,22 @@ __global__ __launch_bounds__(64 * kChWaves) void k_tri_chunk(const TriArgs<T> a)
 }
 
 // The dependency-driven form, for matrices whose rows read scattered rows
-// (kFlowBetter): hardly any dependency stays inside a
-// chunk there, and what bounds the sweep is the number of values fetched.
-// Persistent waves take 64 consecutive level-order positions at a time from
-// a ticket counter and each lane computes its row as soon as the rows it
-// reads are written.  A lane loads its entries eight at a time (plain loads)
-// and consumes them strictly in the row's order; at the first one still
-// kEmpty it polls that one entry with a device-coherent atomic read (a plain
-// load may keep seeing a cached copy) until it is written, then goes on, so
-// the arithmetic is the serial sweep's.  Rows only read rows of earlier
-// levels, which sit at earlier positions, so their tickets were taken by
-// waves that are already running: the sweep cannot deadlock.  A lane that
-// has consumed none of its row's entries for kSpinTicks gives up: it
-// publishes NaN and raises the plan's stall flag (ticket[1]), so the kernel
-// always ends and the solver returns MGX_ERR_TIMEOUT.  At most 1024 waves x
-// 64 rows are in flight, so a valid plan's longest wait is 65536 dependency
-// hops (measured 4-7 us each), far inside the 2 s limit.
+// (kFlowBetter): hardly any dependency stays inside a chunk there, and what
+// bounds the sweep is the number of values fetched. Persistent waves take 64
+// consecutive level-order positions at a time from a ticket counter and each
+// lane computes its row as soon as the rows it reads are written.  A lane
+// loads its entries eight at a time (plain loads) and consumes them strictly
+// in the row's order; at the first one still kEmpty it polls that one entry
+// with a device-coherent atomic read (a plain load may keep seeing a cached
+// copy) until it is written, then goes on, so the arithmetic is the serial
+// sweep's. Rows only read rows of earlier levels, which sit at earlier
+// positions, so their tickets were taken by waves that are already running:
+// the sweep cannot deadlock.  A lane that has consumed none of its row's
+// entries for kSpinTicks gives up: it publishes NaN and raises the plan's
+// stall flag (ticket[1]), so the kernel always ends and the solver returns
+// MGX_ERR_TIMEOUT. At most 1024 waves x 64 rows are in flight, so a valid
+// plan's longest wait is 65536 dependency hops (measured 4-7 us each), far
+// inside the 2 s limit.
 constexpr int kFlowThreads = 256;
 constexpr int kFlowBlocks = 256;
 constexpr int kTriChunk = 8;
