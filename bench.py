@@ -922,6 +922,8 @@ def main():
         "data": "synthetic (generated matrices and seeded U[-1,1) vectors)",
         "config": {"workload": "SpMV (blas::matvec) on the 3D 7-point Laplacian 192^3, FP64, "
                                "CRS int32 indices, n=7077888, nnz=49324032",
+                   "value_counts": "bytes of the CRS arrays, x and y; columns that come from "
+                                   "row patterns are not read, see roofline.bytes_per_launch",
                    "timed_region_s": round(wall, 3)},
         "roofline": roofline,
     }
