@@ -86,6 +86,9 @@ constexpr double kScattered = 0.42, kFlowBetter = 0.6, kFlowLevelUs = 3.6;
 // chunk and from another wave of the chunk, in us
 constexpr double kBatchUs = 0.73, kLevelUs = 0.11, kEntryUs = 0.023, kFarUs = 2.8, kNearUs = 0.09;
 constexpr uint64_t kSpinTicks = 200000000;  // 2 s of the 100 MHz clock without progress
+// 10 ms: a longer gap between two looks at the clock counts as this (nothing
+// ran in it: the process was taken off the device)
+constexpr uint64_t kSpinGap = 1000000;
 
 // batch header: x, y = lanes whose row starts a level, z = rows | values of
 // earlier chunks << 8 | kPart... (a batch with part of its rows' entries:
@@ -140,19 +143,19 @@ __global__ __launch_bounds__(kBlock) void k_tri_init(int64_t n, const int32_t *_
 // wave then gives up (its rows become NaN) and ticket[1] makes the solver
 // return MGX_ERR_TIMEOUT, so every wait ends.
 struct SpinWatch {
-  uint64_t t0 = 0;
+  uint64_t last = 0, waited = 0;
   uint32_t seen = 0, spins = 0;
   __device__ __forceinline__ bool give_up(uint32_t *ticket) {
     if (__builtin_expect((++spins & 255u) != 0, 1)) return false;
     const uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane(
         (int)__hip_atomic_load(ticket + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     const uint64_t now = wall_clock64();
-    if (spins == 256u || p != seen) {
-      seen = p;
-      t0 = now;
-      return false;
-    }
-    if (now - t0 <= kSpinTicks &&
+    const bool moved = spins == 256u || p != seen;
+    waited = moved ? 0 : waited + min(now - last, kSpinGap);
+    last = now;
+    seen = p;
+    if (moved) return false;
+    if (waited <= kSpinTicks &&
         __hip_atomic_load(ticket + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
       return false;
     __hip_atomic_store(ticket + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -439,7 +442,7 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
     const int32_t d1 = has ? rc.z : rc.y;
     const T init = has ? isc[2 * (int64_t)k] : (T)0;
     Acc acc = FIN == 1 ? (Acc)0 : (Acc)init;
-    uint64_t t0 = wall_clock64();  // the lane's last progress
+    uint64_t last = wall_clock64(), waited = 0;  // since the lane's last progress
     int32_t wc = -1;  // >= 0: column of entry d, which was still kEmpty
     T wa = (T)0;
     // a lane publishes its row as soon as its last entry is consumed: a row
@@ -458,7 +461,7 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
               acc = acc - p;
             d++;
             wc = -1;
-            t0 = wall_clock64();
+            waited = 0;
           }
         } else {
           int32_t c[kTriChunk];
@@ -496,9 +499,12 @@ __global__ __launch_bounds__(kFlowThreads) void k_tri_flow(
             }
           }
           d += taken;
-          if (taken > 0) t0 = wall_clock64();
+          if (taken > 0) waited = 0;
         }
-        if (d < d1 && wc >= 0 && wall_clock64() - t0 > kSpinTicks) {
+        const uint64_t now = wall_clock64();
+        waited += min(now - last, kSpinGap);
+        last = now;
+        if (d < d1 && wc >= 0 && waited > kSpinTicks) {
           acc = (Acc)__builtin_bit_cast(T, SweepBits<T>::kNan);
           d = d1;
           __hip_atomic_store(ticket + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
